@@ -328,4 +328,8 @@ int wgrad_check_args(const void* a, const void* b, int64_t B, int64_t K, int64_t
                      int64_t lda, int64_t ldb, int layout, int dtype, const void* out,
                      int64_t ldo, int out_dtype, const float* norms, int flags);
 
+// The least workspace fdp_wgrad_clip accepts for the shape (checked arguments;
+// the size query may ask for more: fp32 calls use it to split their sum pass).
+size_t wgrad_least_workspace(int64_t B, int64_t K, int64_t M, int64_t N, int flags);
+
 }  // namespace fdp

@@ -9,14 +9,15 @@
 // materialises every G_b in HBM and scales it in a second kernel; here no
 // per-sample gradient ever leaves the register file.
 //
-// Three schedules, chosen per call:
+// Four schedules, chosen per call:
 //   single pass (wgrad_core.hpp): 16-bit TN operands whose 128x128 output tiles
 //     fit the co-resident grid: every per-sample tile product stays in the
 //     register file across one grid barrier.
 //   streamed two-pass (wgrad_stream.hpp): the other 16-bit TN problems with
 //     aligned rows (layers larger than the resident grid): Gram-form or direct
 //     per-sample norms, then one clipped-sum contraction per output tile.
-//   generic two-pass (below): fp32 inputs, NN layout, unaligned rows --
+//   fp32 two-pass (wgrad_f32.hpp): fp32 operands of either layout.
+//   generic two-pass (below): 16-bit operands in the NN layout or with unaligned rows --
 //   pass A (wgrad_norm_kernel): one workgroup per (output tile, sample) runs the
 //     tile product on MFMA, squares and sums its fp32 accumulators and writes
 //     one partial per (sample, tile) -- a deterministic [B, tiles] buffer.
@@ -30,8 +31,7 @@
 //     wgrad_finalize_kernel sums in fixed group order.
 //
 // Generic tiles: 128x128 outputs per 256-thread workgroup (4 waves, 64x64 each as 2x2
-// blocks of 32x32 MFMA).  16-bit inputs use v_mfma_f32_32x32x16_{bf16,f16} with
-// BK=64; fp32 inputs use v_mfma_f32_32x32x2_f32 with BK=16.  Global loads are
+// blocks of 32x32 MFMA), v_mfma_f32_32x32x16_{bf16,f16} with BK=64.  Global loads are
 // 16-byte and coalesced along the contiguous dimension; for operands whose
 // contraction axis is strided (every TN operand) the 16-bit loader transposes
 // 4x8 element blocks in registers (v_perm_b32) so that each MFMA lane then reads
@@ -44,6 +44,7 @@
 #include "wgrad_stream.hpp"
 #include <tuple>
 
+#include "wgrad_f32.hpp"
 #include "wgrad_wide.hpp"
 
 namespace fdp {
@@ -170,19 +171,66 @@ __global__ __launch_bounds__(NT) void wgrad_sum_kernel(Args p) {
 }
 
 // out = out_scale * sum_g group_out[g] + noise_scale * noise, fixed order in g.
+// Memory-bound (groups fp32 reads and one write per output): a thread takes 4
+// consecutive outputs, one 16-byte load per group and one Philox block.
+template <class OT>
 __global__ __launch_bounds__(NT) void wgrad_finalize_kernel(Args p) {
+  using S = typename OT::storage;
   const int64_t MN = p.M * p.N;
   const NoiseSrc nz = p.noise.resolved();
-  for (int64_t e = int64_t(blockIdx.x) * NT + threadIdx.x; e < MN; e += int64_t(gridDim.x) * NT) {
-    float s = 0.f;
-    for (int g = 0; g < p.groups; ++g) s += p.group_out[int64_t(g) * MN + e];
-    float v = s * p.out_scale;
-    if (nz.on()) v += p.noise_scale * nz.at(e);
-    const int64_t m = e / p.N, n = e - m * p.N;
-    store_from_f32(p.out, m * p.ldo + n, p.out_dtype, v);
+  S* out = static_cast<S*>(p.out);
+  for (int64_t e = 4 * (int64_t(blockIdx.x) * NT + threadIdx.x); e < MN;
+       e += 4 * int64_t(gridDim.x) * NT) {
+    const int64_t left = MN - e;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    for (int g = 0; g < p.groups; ++g) v += load_quad(p.group_out + int64_t(g) * MN + e, left);
+    v *= p.out_scale;
+    if (nz.draw) {
+      float z[4];
+      nz.block(e / 4, z);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] += p.noise_scale * z[j];
+    } else if (nz.z != nullptr) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (j < left) v[j] += p.noise_scale * nz.at(e + j);
+    }
+    int64_t m = e / p.N, n = e - m * p.N;
+    if (left >= 4 && n + 4 <= p.N) {
+      const S q[4] = {OT::from_f32(v[0]), OT::from_f32(v[1]), OT::from_f32(v[2]), OT::from_f32(v[3])};
+      __builtin_memcpy(out + m * p.ldo + n, q, sizeof(q));
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (j >= left) break;
+        out[m * p.ldo + n] = OT::from_f32(v[j]);
+        if (++n == p.N) {
+          n = 0;
+          ++m;
+        }
+      }
+    }
   }
 }
 
+void launch_factors(const Args& a, int per_sample, bool noclip, hipStream_t s) {
+  const unsigned fb = static_cast<unsigned>((a.B + (NT / kWave) - 1) / (NT / kWave));
+  hipLaunchKernelGGL(wgrad_factor_kernel, dim3(fb < 1024 ? fb : 1024), dim3(NT), 0, s, a.partials,
+                     a.B, per_sample, a.C, a.clamp, a.clip_args_dev, noclip ? 1 : 0,
+                     const_cast<float*>(a.factors), a.norms_out, a.factors_out, a.err);
+}
+
+void launch_finalize(const Args& a, hipStream_t s) {
+  int64_t nb = (a.M * a.N + 4 * NT - 1) / (4 * NT);
+  if (nb > 4096) nb = 4096;
+  const dim3 grid(static_cast<unsigned>(nb));
+  if (a.out_dtype == FDP_BF16)
+    hipLaunchKernelGGL(wgrad_finalize_kernel<BF16>, grid, dim3(NT), 0, s, a);
+  else if (a.out_dtype == FDP_F16)
+    hipLaunchKernelGGL(wgrad_finalize_kernel<F16>, grid, dim3(NT), 0, s, a);
+  else
+    hipLaunchKernelGGL(wgrad_finalize_kernel<F32>, grid, dim3(NT), 0, s, a);
+}
 
 }  // namespace wg
 }  // namespace fdp
@@ -296,52 +344,70 @@ Plan cached_plan(int64_t B, int64_t K, int64_t M, int64_t N, int cus, int flags,
                    [&] { return make_plan(B, K, M, N, cus, flags, lda, ldb); });
 }
 
+// Workspace of the fp32 schedule: partials [B, per_sample], factors [B], group
+// partials [splits, M, N].
+struct F32Layout {
+  F32Plan plan;
+  size_t off_partials, off_factors, off_group, total;
+};
+
+// Splits of the fp32 sum pass: their partials stay below one fp32 gradient per
+// sample or 32 MB, whichever is more, and below 256 MB.  lean: the plan that
+// fits a workspace of make_plan's size (old_groups group partials).
+F32Layout f32_layout(int64_t B, int64_t K, int64_t M, int64_t N, int layout, int cus,
+                     int old_groups, bool lean) {
+  using Key = std::tuple<int64_t, int64_t, int64_t, int64_t, int, int, int, bool>;
+  static host::ShapeCache<Key, F32Layout> cache;
+  return cache.get(Key{B, K, M, N, layout, cus, old_groups, lean}, [&] {
+    F32Layout l{};
+    const double mn = 4. * double(M) * double(N);
+    int64_t most = old_groups;
+    if (!lean) {
+      const double bytes = double(B) * mn > 32e6 ? double(B) * mn : 32e6;
+      most = static_cast<int64_t>((bytes < 256e6 ? bytes : 256e6) / mn);
+      if (most < old_groups) most = old_groups;
+    }
+    l.plan = f32_plan(B, K, M, N, layout, cus, most, lean);
+    l.off_partials = kWsHead;
+    l.off_factors =
+        l.off_partials + align_up(sizeof(float) * size_t(B) * size_t(l.plan.per_sample));
+    l.off_group = l.off_factors + align_up(sizeof(float) * size_t(B));
+    l.total = l.off_group;
+    if (l.plan.splits > 1)
+      l.total += align_up(sizeof(float) * size_t(l.plan.splits) * size_t(M) * size_t(N));
+    return l;
+  });
+}
+
 template <class Core, int LAYOUT, bool VEC>
-hipError_t launch_passes(const Args& a, const Plan& pl, bool noclip, float C, float clamp,
-                         const float* clip_args_dev, float* norms, float* factors, float* fac_ws,
-                         hipStream_t s) {
+hipError_t launch_passes(const Args& a, const Plan& pl, bool noclip, hipStream_t s) {
   const dim3 block(NT);
   if (!noclip) {
     hipLaunchKernelGGL((wgrad_norm_kernel<Core, LAYOUT, VEC>), dim3(pl.tiles, a.B), block,
                        Core::SMEM, s, a);
   }
-  const unsigned fb = static_cast<unsigned>((a.B + (NT / kWave) - 1) / (NT / kWave));
-  hipLaunchKernelGGL(wgrad_factor_kernel, dim3(fb < 1024 ? fb : 1024), block, 0, s, a.partials,
-                     a.B, pl.tiles, C, clamp, clip_args_dev, noclip ? 1 : 0, fac_ws, norms,
-                     factors, a.err);
+  launch_factors(a, pl.tiles, noclip, s);
   hipLaunchKernelGGL((wgrad_sum_kernel<Core, LAYOUT, VEC>), dim3(pl.tiles, pl.groups), block,
                      Core::SMEM, s, a);
-  if (pl.groups > 1) {
-    const int64_t MN = a.M * a.N;
-    int64_t nb = (MN + NT - 1) / NT;
-    if (nb > 4096) nb = 4096;
-    hipLaunchKernelGGL(wgrad_finalize_kernel, dim3(static_cast<unsigned>(nb)), block, 0, s, a);
-  }
+  if (pl.groups > 1) launch_finalize(a, s);
   return hipGetLastError();
 }
 
 template <class Core>
 hipError_t dispatch_layout(int layout, bool vec, const Args& a, const Plan& pl, bool noclip,
-                           float C, float clamp, const float* cad, float* norms, float* factors,
-                           float* fac_ws, hipStream_t s) {
+                           hipStream_t s) {
   if (layout == FDP_LAYOUT_TN) {
-    return vec ? launch_passes<Core, FDP_LAYOUT_TN, true>(a, pl, noclip, C, clamp, cad, norms,
-                                                          factors, fac_ws, s)
-               : launch_passes<Core, FDP_LAYOUT_TN, false>(a, pl, noclip, C, clamp, cad, norms,
-                                                           factors, fac_ws, s);
+    return vec ? launch_passes<Core, FDP_LAYOUT_TN, true>(a, pl, noclip, s)
+               : launch_passes<Core, FDP_LAYOUT_TN, false>(a, pl, noclip, s);
   }
-  return vec ? launch_passes<Core, FDP_LAYOUT_NN, true>(a, pl, noclip, C, clamp, cad, norms,
-                                                        factors, fac_ws, s)
-             : launch_passes<Core, FDP_LAYOUT_NN, false>(a, pl, noclip, C, clamp, cad, norms,
-                                                         factors, fac_ws, s);
+  return vec ? launch_passes<Core, FDP_LAYOUT_NN, true>(a, pl, noclip, s)
+             : launch_passes<Core, FDP_LAYOUT_NN, false>(a, pl, noclip, s);
 }
 
 // Streamed two-pass schedule for 16-bit TN operands with aligned rows: Gram
 // (or direct) norms, factors, then one clipped-sum contraction per output tile.
 template <class DT>
-hipError_t launch_stream(Args a, const Plan& pl, bool noclip, float C, float clamp,
-                         const float* clip_args_dev, float* norms, float* factors, float* fac_ws,
-                         hipStream_t s) {
+hipError_t launch_stream(Args a, const Plan& pl, bool noclip, hipStream_t s) {
   const dim3 block(NT);
   int per_sample = pl.tiles;
   if (!noclip) {
@@ -375,25 +441,14 @@ hipError_t launch_stream(Args a, const Plan& pl, bool noclip, float C, float cla
   a.fac_parts = 0;
   if (!noclip && pl.sp.sum_spg <= kSumFacMax) {
     a.fac_parts = per_sample;
-    a.C = C;
-    a.clamp = clamp;
-    a.clip_args_dev = clip_args_dev;
-    a.norms_out = norms;
-    a.factors_out = factors;
   } else {
-    const unsigned fb = static_cast<unsigned>((a.B + (NT / kWave) - 1) / (NT / kWave));
-    hipLaunchKernelGGL(wgrad_factor_kernel, dim3(fb < 1024 ? fb : 1024), block, 0, s, a.partials,
-                       a.B, per_sample, C, clamp, clip_args_dev, noclip ? 1 : 0, fac_ws, norms,
-                       factors, a.err);
+    launch_factors(a, per_sample, noclip, s);
   }
   const hipError_t e = DT::code == FDP_BF16 ? launch_clipsum_bf16(a, pl.sp, s) : launch_clipsum_f16(a, pl.sp, s);
   if (e != hipSuccess) return e;
   if (pl.sp.sum_groups > 1) {
     a.groups = pl.sp.sum_groups;
-    const int64_t MN = a.M * a.N;
-    int64_t nb = (MN + NT - 1) / NT;
-    if (nb > 4096) nb = 4096;
-    hipLaunchKernelGGL(wgrad_finalize_kernel, dim3(static_cast<unsigned>(nb)), block, 0, s, a);
+    launch_finalize(a, s);
   }
   return hipGetLastError();
 }
@@ -406,8 +461,20 @@ extern "C" int fdp_wgrad_clip_workspace_size(int64_t B, int64_t K, int64_t M, in
   if (bytes == nullptr) return FDP_ERR_ARG;
   if (!valid_dtype(dtype)) return FDP_ERR_DTYPE;
   if (B < 1 || M < 1 || N < 1 || K < 0) return FDP_ERR_SHAPE;
-  *bytes = cached_plan(B, K, M, N, num_cus(), flags).total;
+  const int cus = num_cus();
+  const Plan pl = cached_plan(B, K, M, N, cus, flags);
+  *bytes = pl.total;
+  if (dtype == FDP_F32) {
+    for (int layout : {FDP_LAYOUT_TN, FDP_LAYOUT_NN}) {
+      const size_t t = f32_layout(B, K, M, N, layout, cus, pl.groups, false).total;
+      if (t > *bytes) *bytes = t;
+    }
+  }
   return FDP_OK;
+}
+
+size_t fdp::wgrad_least_workspace(int64_t B, int64_t K, int64_t M, int64_t N, int flags) {
+  return cached_plan(B, K, M, N, num_cus(), flags).total;
 }
 
 int fdp::wgrad_check_args(const void* a, const void* b, int64_t B, int64_t K, int64_t M,
@@ -633,24 +700,28 @@ int wgrad_clip_impl(const void* a, const void* b, int64_t B, int64_t K, int64_t 
   if (layout == FDP_LAYOUT_TN && vec && dtype != FDP_F32 && K > 0 && fits_record(K, lda) &&
       fits_record(K, ldb)) {
     args.group_out = pl.sp.sum_groups > 1 ? reinterpret_cast<float*>(ws + pl.off_group) : nullptr;
-    e = dtype == FDP_BF16 ? launch_stream<BF16>(args, pl, noclip, C, clamp, clip_args_dev, norms,
-                                                factors, fac_ws, s)
-                          : launch_stream<F16>(args, pl, noclip, C, clamp, clip_args_dev, norms,
-                                               factors, fac_ws, s);
+    e = dtype == FDP_BF16 ? launch_stream<BF16>(args, pl, noclip, s)
+                          : launch_stream<F16>(args, pl, noclip, s);
     if (e != hipSuccess) return FDP_ERR_HIP;
     if (bias_done != nullptr) *bias_done = bias != nullptr;
     return FDP_OK;
   }
   args.bias_op = 0;  // the generic schedule: the caller forms the bias
-  if (dtype == FDP_BF16) {
-    e = dispatch_layout<Core16<BF16>>(layout, vec, args, pl, noclip, C, clamp, clip_args_dev,
-                                      norms, factors, fac_ws, s);
-  } else if (dtype == FDP_F16) {
-    e = dispatch_layout<Core16<F16>>(layout, vec, args, pl, noclip, C, clamp, clip_args_dev,
-                                     norms, factors, fac_ws, s);
+  if (dtype == FDP_F32) {
+    // the plan that the workspace query sized, or, in a smaller workspace, the
+    // one that fits the least accepted size
+    const F32Layout fl = f32_layout(B, K, M, N, layout, cus, pl0.groups, false);
+    const F32Layout f = fl.total <= workspace_bytes
+                            ? fl
+                            : f32_layout(B, K, M, N, layout, cus, pl0.groups, true);
+    args.partials = reinterpret_cast<float*>(ws + f.off_partials);
+    args.factors = reinterpret_cast<float*>(ws + f.off_factors);
+    args.group_out = reinterpret_cast<float*>(ws + f.off_group);
+    e = launch_f32(args, f.plan, layout, noclip, s);
+  } else if (dtype == FDP_BF16) {
+    e = dispatch_layout<Core16<BF16>>(layout, vec, args, pl, noclip, s);
   } else {
-    e = dispatch_layout<Core32>(layout, vec, args, pl, noclip, C, clamp, clip_args_dev, norms,
-                                factors, fac_ws, s);
+    e = dispatch_layout<Core16<F16>>(layout, vec, args, pl, noclip, s);
   }
   return e == hipSuccess ? FDP_OK : FDP_ERR_HIP;
 }
@@ -680,11 +751,13 @@ namespace {
 struct BiasLayout {
   size_t wspan, col_off, part_off, sq_off, total;
 };
+// least: with the smallest weight workspace that is accepted.
 int bias_layout(int64_t B, int64_t K, int64_t M, int64_t N, int dtype, int wflags, int bias_op,
-                BiasLayout* l) {
+                bool least, BiasLayout* l) {
   size_t w = 0, c = 0;
   int st = fdp_wgrad_clip_workspace_size(B, K, M, N, dtype, wflags, &w);
   if (st != FDP_OK) return st;
+  if (least) w = fdp::wgrad_least_workspace(B, K, M, N, wflags);
   st = fdp_colsum_clip_workspace_size(B, K, bias_op == 1 ? M : N, dtype, &c);
   if (st != FDP_OK) return st;
   const int gm = static_cast<int>((M + BM - 1) / BM), gn = static_cast<int>((N + BN - 1) / BN);
@@ -711,7 +784,7 @@ extern "C" int fdp_wgrad_bias_clip_workspace_size(int64_t B, int64_t K, int64_t 
   if (B < 1 || M < 1 || N < 1 || K < 0) return FDP_ERR_SHAPE;
   const int bias_op = (flags & FDP_WGRAD_BIAS_OF_B) ? 2 : 1;
   BiasLayout l{};
-  const int st = bias_layout(B, K, M, N, dtype, flags & ~FDP_WGRAD_BIAS_OF_B, bias_op, &l);
+  const int st = bias_layout(B, K, M, N, dtype, flags & ~FDP_WGRAD_BIAS_OF_B, bias_op, false, &l);
   if (st != FDP_OK) return st;
   *bytes = l.total;
   return FDP_OK;
@@ -739,7 +812,9 @@ extern "C" int fdp_wgrad_bias_clip(const void* a, const void* b, int64_t B, int6
   if (bias_op == 1 && (lda != M || stride_ab != K * M)) return FDP_ERR_SHAPE;
   if (bias_op == 2 && (ldb != N || stride_bb != K * N)) return FDP_ERR_SHAPE;
   BiasLayout l{};
-  int st = bias_layout(B, K, M, N, dtype, flags, bias_op, &l);
+  int st = bias_layout(B, K, M, N, dtype, flags, bias_op, false, &l);
+  if (st == FDP_OK && workspace_bytes < l.total)
+    st = bias_layout(B, K, M, N, dtype, flags, bias_op, true, &l);
   if (st != FDP_OK) return st;
   if (workspace == nullptr || workspace_bytes < l.total) return FDP_ERR_WORKSPACE;
   char* ws = static_cast<char*>(workspace);

@@ -248,136 +248,6 @@ struct Core16 {
   }
 };
 
-// ------------------------------------------------------------------- fp32
-// LDS tile: [16 k][128 r] floats, row stride 132 floats; MFMA 32x32x2 reads one
-// float per lane per operand, consecutive lanes on consecutive r.
-struct Core32 {
-  static constexpr int BK = 16;
-  static constexpr int LD = 132;
-  static constexpr int TILE_BYTES = BK * LD * 4;
-  static constexpr int SMEM = 4 * TILE_BYTES;
-
-  template <bool VEC>
-  __device__ static inline void load_kr(const float* src, int64_t ld, int64_t K, int64_t R,
-                                        int64_t k0, int64_t r0, float4 (&reg)[2]) {
-    const int t = threadIdx.x;
-    const int64_t k = k0 + (t >> 4);
-    const int64_t r = r0 + (t & 15) * 8;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-      const int64_t ri = r + 4 * i;
-      if (k < K) {
-        const float* p = src + k * ld + ri;
-        if (VEC && ri + 4 <= R) {
-          v = *reinterpret_cast<const float4*>(p);
-        } else {
-          v.x = (ri + 0 < R) ? p[0] : 0.f;
-          v.y = (ri + 1 < R) ? p[1] : 0.f;
-          v.z = (ri + 2 < R) ? p[2] : 0.f;
-          v.w = (ri + 3 < R) ? p[3] : 0.f;
-        }
-      }
-      reg[i] = v;
-    }
-  }
-  __device__ static inline void store_kr(char* lds, const float4 (&reg)[2]) {
-    const int t = threadIdx.x;
-    float* base = reinterpret_cast<float*>(lds) + (t >> 4) * LD + (t & 15) * 8;
-    *reinterpret_cast<float4*>(base) = reg[0];
-    *reinterpret_cast<float4*>(base + 4) = reg[1];
-  }
-  // [R, K] with K contiguous: thread t loads row r0+(t>>1), k = k0+8*(t&1)..+7.
-  template <bool VEC>
-  __device__ static inline void load_rk(const float* src, int64_t ld, int64_t K, int64_t R,
-                                        int64_t k0, int64_t r0, float4 (&reg)[2]) {
-    const int t = threadIdx.x;
-    const int64_t r = r0 + (t >> 1);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int64_t k = k0 + (t & 1) * 8 + 4 * i;
-      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (r < R) {
-        const float* p = src + r * ld + k;
-        if (VEC && k + 4 <= K) {
-          v = *reinterpret_cast<const float4*>(p);
-        } else {
-          v.x = (k + 0 < K) ? p[0] : 0.f;
-          v.y = (k + 1 < K) ? p[1] : 0.f;
-          v.z = (k + 2 < K) ? p[2] : 0.f;
-          v.w = (k + 3 < K) ? p[3] : 0.f;
-        }
-      }
-      reg[i] = v;
-    }
-  }
-  __device__ static inline void store_rk(char* lds, const float4 (&reg)[2]) {
-    const int t = threadIdx.x;
-    float* base = reinterpret_cast<float*>(lds) + (t >> 1);
-    const int kb = (t & 1) * 8;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      base[(kb + 4 * i + 0) * LD] = reg[i].x;
-      base[(kb + 4 * i + 1) * LD] = reg[i].y;
-      base[(kb + 4 * i + 2) * LD] = reg[i].z;
-      base[(kb + 4 * i + 3) * LD] = reg[i].w;
-    }
-  }
-  __device__ static inline void mma(const char* As, const char* Bs, f32x16 (&acc)[2][2], int wm,
-                                    int wn, int lane) {
-    const float* A = reinterpret_cast<const float*>(As);
-    const float* Bf = reinterpret_cast<const float*>(Bs);
-    const int rr = lane & 31;
-#pragma unroll
-    for (int ks = 0; ks < BK / 2; ++ks) {
-      const int k = ks * 2 + (lane >> 5);
-      const float a0 = A[k * LD + wm + rr], a1 = A[k * LD + wm + 32 + rr];
-      const float b0 = Bf[k * LD + wn + rr], b1 = Bf[k * LD + wn + 32 + rr];
-      acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b0, acc[0][0], 0, 0, 0);
-      acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b1, acc[0][1], 0, 0, 0);
-      acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b0, acc[1][0], 0, 0, 0);
-      acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b1, acc[1][1], 0, 0, 0);
-    }
-  }
-  template <int LAYOUT, bool VEC>
-  __device__ static void gemm(const Args& p, int64_t bidx, int64_t m0, int64_t n0,
-                              f32x16 (&acc)[2][2], char* smem) {
-    const float* A = static_cast<const float*>(p.a) + bidx * p.sab;
-    const float* Bm = static_cast<const float*>(p.b) + bidx * p.sbb;
-    // Buffer c holds the A tile at smem + 2c*TILE_BYTES and the B tile right after.
-#define FDP_AS(c) (smem + (c) * (2 * TILE_BYTES))
-#define FDP_BS(c) (smem + (c) * (2 * TILE_BYTES) + TILE_BYTES)
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-    const int nk = static_cast<int>((p.K + BK - 1) / BK);
-    float4 ra[2], rb[2];
-    if (LAYOUT == FDP_LAYOUT_TN) load_kr<VEC>(A, p.lda, p.K, p.M, 0, m0, ra);
-    else load_rk<VEC>(A, p.lda, p.K, p.M, 0, m0, ra);
-    load_kr<VEC>(Bm, p.ldb, p.K, p.N, 0, n0, rb);
-    if (LAYOUT == FDP_LAYOUT_TN) store_kr(FDP_AS(0), ra);
-    else store_rk(FDP_AS(0), ra);
-    store_kr(FDP_BS(0), rb);
-    __syncthreads();
-    for (int kt = 0; kt < nk; ++kt) {
-      const int cur = kt & 1;
-      const bool more = kt + 1 < nk;
-      if (more) {
-        const int64_t k0 = int64_t(kt + 1) * BK;
-        if (LAYOUT == FDP_LAYOUT_TN) load_kr<VEC>(A, p.lda, p.K, p.M, k0, m0, ra);
-        else load_rk<VEC>(A, p.lda, p.K, p.M, k0, m0, ra);
-        load_kr<VEC>(Bm, p.ldb, p.K, p.N, k0, n0, rb);
-      }
-      mma(FDP_AS(cur), FDP_BS(cur), acc, wm, wn, lane);
-      if (more) {
-        if (LAYOUT == FDP_LAYOUT_TN) store_kr(FDP_AS(cur ^ 1), ra);
-        else store_rk(FDP_AS(cur ^ 1), ra);
-        store_kr(FDP_BS(cur ^ 1), rb);
-      }
-      __syncthreads();
-    }
-  }
-};
-
 #undef FDP_AS
 #undef FDP_BS
 

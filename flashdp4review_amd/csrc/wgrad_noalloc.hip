@@ -77,9 +77,7 @@ extern "C" int fdp_wgrad_clip_noalloc(const void* a, const void* b, int64_t B, i
   // The control words are cleared by the call itself (a small fill kernel):
   // an expired wait of an earlier call may have left its status word set.
   flags = (flags | FDP_WGRAD_PLAIN_LAUNCH) & ~FDP_WGRAD_CLEAN_WORKSPACE;
-  size_t need = 0;
-  const int st = fdp_wgrad_clip_workspace_size(B, K, M, N, dtype, flags, &need);
-  if (st != FDP_OK) return st;
+  const size_t need = fdp::wgrad_least_workspace(B, K, M, N, flags);
   if (need > size_t(FDP_NOALLOC_SCRATCH_BYTES)) return FDP_ERR_TOO_LARGE;
   void* ws = device_scratch();
   if (ws == nullptr) return FDP_ERR_HIP;

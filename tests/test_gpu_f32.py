@@ -1,0 +1,125 @@
+"""The fp32 two-pass schedule (csrc/wgrad_f32.hpp) at the edges of its rules.
+
+Against the float64 oracle at the repository's fp32 bar (1e-5): samples of one
+row (||a||^2 ||b||^2), of 2..16 rows (fp64 row-Gram norms or direct ones, by
+cost), 17 rows and more (direct); k-tiles that hold rows of several samples;
+64- and 128-wide tiles with ragged edges; split contractions; more samples per
+workgroup than it forms factors for; both layouts.
+"""
+import numpy as np
+import pytest
+import torch
+
+from oracle import dp_clip as O
+from oracle import philox
+from tests._tol import assert_close, assert_elementwise
+
+from flashdp4review_amd import _lib, core
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+SHAPES = [  # B, K, M, N
+    (1, 1, 1, 1),           # one value
+    (5, 1, 70, 129),        # one row a sample, ragged 64-wide tiles
+    (300, 1, 256, 320),     # several samples in every k-tile
+    (2500, 1, 64, 64),      # more samples than a workgroup's factor table
+    (7, 2, 131, 67),        # row Gram or direct, samples straddle k-tiles
+    (64, 3, 512, 640),
+    (33, 16, 640, 512),     # the row Gram's longest sample
+    (33, 17, 320, 256),     # one row more: direct norms
+    (3, 50, 70, 90),
+    (4, 128, 768, 768),
+    (2, 700, 300, 260),     # split contraction, rows not a multiple of a k-tile
+    (8, 96, 1100, 1030),    # 128-wide tiles, ragged both ways
+    (1, 4096, 129, 65),     # one long sample
+]
+
+
+def make(B, K, M, N, layout, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    a = torch.randn((B, K, M) if layout == "tn" else (B, M, K), generator=g)
+    b = torch.randn(B, K, N, generator=g) * (0.1 + torch.rand(B, 1, 1, generator=g))
+    return a.to(DEV), b.to(DEV)
+
+
+@pytest.mark.parametrize("layout", ["tn", "nn"])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_f32_parity(shape, layout):
+    B, K, M, N = shape
+    a, b = make(B, K, M, N, layout)
+    _, norms_ref, _ = O.wgrad_clip(a, b, 1.0, 1.0, layout)
+    C = float(np.median(norms_ref)) * (1.0 if B > 1 else 0.5)
+    ref, norms_ref, fac_ref = O.wgrad_clip(a, b, C, 1.0, layout)
+    out, norms, fac = core.wgrad_clip(a, b, C, 1.0, layout=layout, return_stats=True)
+    assert_close(out, ref, torch.float32, "sum")
+    assert_elementwise(norms, norms_ref, torch.float32, "norms")
+    assert_elementwise(fac, fac_ref, torch.float32, "factors")
+    assert torch.equal(out, core.wgrad_clip(a, b, C, 1.0, layout=layout))
+
+
+@pytest.mark.parametrize("K", [1, 2, 16])
+def test_f32_cancelling_rows(K):
+    """Rows that cancel: every pair's sum is 1e-3 of its terms, so the squared
+    norm is 1e-6 of the Gram terms it is summed from (2e-16 each in fp64,
+    6e-8 in fp32); the bound is the 1e-5 bar over the 1e-3 that fp32 inputs keep."""
+    B, M, N = 6, 96, 160
+    g = torch.Generator().manual_seed(4)
+    a = torch.randn(B, K, M, generator=g)
+    x = torch.randn(B, 1, N, generator=g).expand(B, K, N).contiguous()
+    for k in range(1, K, 2):
+        a[:, k] = -a[:, k - 1] * (1 + 1e-3)
+    _, norms_ref, _ = O.wgrad_clip(a, x, 1.0, 1.0, "tn")
+    _, norms, _ = core.wgrad_clip(a.to(DEV), x.to(DEV), 1.0, 1.0, return_stats=True)
+    e = np.abs(norms.double().cpu().numpy() - norms_ref) / norms_ref
+    assert e.max() <= 1e-5
+
+
+@pytest.mark.parametrize("shape", [(6, 1, 96, 100), (6, 20, 96, 101)], ids=lambda s: "x".join(map(str, s)))
+def test_f32_infinite_sample_is_left_out(shape):
+    """A sample with an infinite entry in a has an infinite norm, so its factor
+    is zero and it adds nothing, although its neighbours share its k-tiles."""
+    B, K, M, N = shape
+    a, b = make(B, K, M, N, "tn", seed=2)
+    b[3] = b[3].abs() + 0.5  # (no zero times infinity in its norm)
+    keep = [i for i in range(B) if i != 3]
+    ref, _, _ = O.wgrad_clip(a[keep], b[keep], 1.0, 1.0, "tn")
+    a[3] = a[3].abs() + 0.5
+    a[3, 0, 5] = float("inf")
+    out, norms, fac = core.wgrad_clip(a, b, 1.0, 1.0, return_stats=True)
+    assert torch.isinf(norms[3]) and float(fac[3]) == 0.0
+    assert_close(out, ref, torch.float32)
+
+
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("shape", [(4, 64, 130, 96), (2, 640, 66, 101)], ids=lambda s: "x".join(map(str, s)))
+def test_f32_noise_strides_and_least_workspace(shape, out_dtype):
+    """The drawn noise in the sum pass's and in the split sum's epilogue, into a
+    strided output, from strided operands; and the call in the least workspace
+    that is accepted (fewer splits)."""
+    B, K, M, N = shape
+    a, b = make(B, K + 3, M + 5, N + 2, "tn", seed=5)
+    a, b = a[:, 1:K + 1, 2:M + 2], b[:, 2:K + 2, 1:N + 1]
+    wide = torch.zeros(M, N + 7, dtype=out_dtype, device=DEV)
+    ref, _, _ = O.wgrad_clip(a, b, 1.0, 0.9, "tn")
+    z = philox.normals(M * N, 77, 5).reshape(M, N)
+    expect = ref / B + 0.01 * z
+    core.wgrad_clip(a, b, 1.0, 0.9, out_scale=1.0 / B, noise_scale=0.01, noise_key=(77, 5),
+                    out=wide[:, 3:N + 3])
+    assert_close(wide[:, 3:N + 3], expect, out_dtype, "strided")
+    assert torch.count_nonzero(wide[:, :3]) == 0 and torch.count_nonzero(wide[:, N + 3:]) == 0
+    a, b = a.contiguous(), b.contiguous()
+    L = _lib.lib()
+    most = _lib.size_query(L.fdp_wgrad_clip_workspace_size, B, K, M, N, _lib.FDP_F32, 0)
+    least = _lib.size_query(L.fdp_wgrad_clip_workspace_size, B, K, M, N, _lib.FDP_BF16, 0)
+    outs = []
+    for nbytes in (most, least):
+        ws = torch.zeros(nbytes, dtype=torch.uint8, device=DEV)
+        out = torch.empty(M, N, device=DEV)
+        st = L.fdp_wgrad_clip(a.data_ptr(), b.data_ptr(), B, K, M, N, K * M, M, K * N, N,
+                              _lib.LAYOUT_TN, _lib.FDP_F32, 1.0, 0.9, None, 1.0 / B, None, 0.0, None,
+                              out.data_ptr(), N, _lib.FDP_F32, None, None, 0, ws.data_ptr(), nbytes,
+                              _lib.stream_handle(torch.device(DEV, torch.cuda.current_device())))
+        assert st == 0
+        outs.append(out)
+        assert_close(out, ref / B, torch.float32, f"{nbytes} bytes")
