@@ -391,14 +391,17 @@ template <class G>
 struct Job {
   Operand<G::LOADS_A, G::BK> a;
   Operand<G::LOADS_B, G::BK> b;
+  // M: operand A's rows where it is k-contiguous (else unused)
   __device__ __forceinline__ void init(const uint16_t* pa, int64_t lda, const uint16_t* pb,
-                                       int64_t ldb, int64_t K, int64_t m0, int64_t n0) {
-    a.template init<G::BM>(pa, lda, K, m0);
+                                       int64_t ldb, int64_t K, int64_t m0, int64_t n0,
+                                       int64_t M = 0) {
+    if constexpr (G::AKC) a.template init_kc<G::BM>(pa, lda, M, m0);
+    else a.template init<G::BM>(pa, lda, K, m0);
     b.template init<G::BN>(pb, ldb, K, n0);
   }
   __device__ __forceinline__ void retarget(const uint16_t* pa, int64_t lda, const uint16_t* pb,
-                                           int64_t ldb, int64_t K) {
-    a.retarget(pa, lda, K);
+                                           int64_t ldb, int64_t K, int64_t M = 0) {
+    a.retarget(pa, lda, G::AKC ? M : K);
     b.retarget(pb, ldb, K);
   }
   __device__ __forceinline__ void retile(int64_t m0, int64_t n0) {

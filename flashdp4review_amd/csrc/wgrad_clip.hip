@@ -10,75 +10,31 @@
 // per-sample gradient ever leaves the register file.
 //
 // Four schedules, chosen per call:
-//   single pass (wgrad_core.hpp): 16-bit TN operands whose 128x128 output tiles
-//     fit the co-resident grid: every per-sample tile product stays in the
-//     register file across one grid barrier.
-//   streamed two-pass (wgrad_stream.hpp): the other 16-bit TN problems with
-//     aligned rows (layers larger than the resident grid): Gram-form or direct
-//     per-sample norms, then one clipped-sum contraction per output tile.
+//   single pass (wgrad_wide.hpp, wgrad_core.hpp): 16-bit TN operands with aligned
+//     rows whose output tiles fit the co-resident grid: every per-sample tile
+//     product stays in the register file across one grid barrier.
+//   streamed two-pass (wgrad_stream.hpp): the other 16-bit problems with aligned
+//     rows (layers larger than the resident grid, the NN layout): per-sample norms
+//     in Gram form or from the products, then one clipped-sum contraction per
+//     output tile.
+//   register-fed two-pass (wgrad_staged.hpp): the same for 16-bit operands the
+//     LDS-DMA core cannot read (unaligned rows, ragged K in the NN layout, samples
+//     past a 32-bit buffer record).
 //   fp32 two-pass (wgrad_f32.hpp): fp32 operands of either layout.
-//   generic two-pass (below): 16-bit operands in the NN layout or with unaligned rows --
-//   pass A (wgrad_norm_kernel): one workgroup per (output tile, sample) runs the
-//     tile product on MFMA, squares and sums its fp32 accumulators and writes
-//     one partial per (sample, tile) -- a deterministic [B, tiles] buffer.
-//   factor (wgrad_factor_kernel): fixed-order sum of each sample's partials ->
-//     ||G_b||, c_b.
-//   pass B (wgrad_sum_kernel): one workgroup per (output tile, sample group)
-//     accumulates the group's samples into ONE fp32 accumulator, rescaling it
-//     by c_prev/c_b at each sample boundary so that it always holds
-//     sum c_b G_b / c_current; the epilogue multiplies by the last c and applies
-//     out_scale and the noise (single group) or writes an fp32 group partial that
-//     wgrad_finalize_kernel sums in fixed group order.
-//
-// Generic tiles: 128x128 outputs per 256-thread workgroup (4 waves, 64x64 each as 2x2
-// blocks of 32x32 MFMA), v_mfma_f32_32x32x16_{bf16,f16} with BK=64.  Global loads are
-// 16-byte and coalesced along the contiguous dimension; for operands whose
-// contraction axis is strided (every TN operand) the 16-bit loader transposes
-// 4x8 element blocks in registers (v_perm_b32) so that each MFMA lane then reads
-// its 8 consecutive k-values with one ds_read_b128.  LDS rows are XOR-swizzled
-// in 16-byte chunks to spread both the transposing writes and the fragment
-// reads over the banks.  LDS is double-buffered: the next k-tile's global loads
-// are issued before the current tile's MFMAs.
+// The two-pass schedules form the clip factors in the sum pass; calls without
+// clipping and very large batches launch wgrad_factor_kernel between the passes,
+// and a split sum ends in wgrad_finalize_kernel.
 #include <cstdlib>
 
 #include "wgrad_stream.hpp"
 #include <tuple>
 
 #include "wgrad_f32.hpp"
+#include "wgrad_staged.hpp"
 #include "wgrad_wide.hpp"
 
 namespace fdp {
 namespace wg {
-
-// ---------------------------------------------------------------- pass A
-template <class Core, int LAYOUT, bool VEC>
-__global__ __launch_bounds__(NT) void wgrad_norm_kernel(Args p) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int tile = blockIdx.x;
-  const int64_t bidx = blockIdx.y;
-  int64_t m0, n0;
-  tile_coords(p, tile, m0, n0);
-  f32x16 acc[2][2];
-  zero(acc);
-  Core::template gemm<LAYOUT, VEC>(p, bidx, m0, n0, acc, smem);
-  // Out-of-range rows/columns were loaded as zeros, so they add nothing.
-  float s = 0.f;
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s += acc[i][j][r] * acc[i][j][r];
-  s = wave_sum(s);
-  float* red = reinterpret_cast<float*>(smem);  // gemm() ended on a barrier
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) red[wave] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const int tiles = p.tiles_m * p.tiles_n;
-    p.partials[bidx * tiles + tile] = (red[0] + red[1]) + (red[2] + red[3]);
-  }
-}
 
 // ---------------------------------------------------------------- factors
 // One wavefront per sample: ||G_b|| = sqrt(sum over tiles of partials[b, :]),
@@ -101,7 +57,8 @@ __global__ __launch_bounds__(NT) void wgrad_factor_kernel(const float* partials,
     if (!noclip) {
       float s = 0.f;
       for (int t = lane; t < tiles; t += kWave) s += partials[b * tiles + t];
-      n = sqrtf(wave_sum(s));
+      s = wave_sum(s);
+      n = sqrtf(s < 0.f ? 0.f : s);  // (a Gram sum may round below zero)
     }
     if (lane == 0) {
       const float c = noclip ? clamp : clip_factor(n, C, clamp);
@@ -110,64 +67,6 @@ __global__ __launch_bounds__(NT) void wgrad_factor_kernel(const float* partials,
       if (factors) factors[b] = c;
     }
   }
-}
-
-// ---------------------------------------------------------------- pass B
-template <class Core, int LAYOUT, bool VEC>
-__global__ __launch_bounds__(NT) void wgrad_sum_kernel(Args p) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int tile = blockIdx.x;
-  const int g = blockIdx.y;
-  int64_t m0, n0;
-  tile_coords(p, tile, m0, n0);
-  const int64_t b_begin = int64_t(g) * p.spg;
-  const int64_t b_end = b_begin + p.spg < p.B ? b_begin + p.spg : p.B;
-
-  f32x16 acc[2][2];
-  zero(acc);
-  float c_prev = 0.f;
-  bool any = false;
-  for (int64_t bidx = b_begin; bidx < b_end; ++bidx) {
-    const float c = p.factors[bidx];
-    if (c == 0.f) continue;  // contributes exactly zero
-    if (any) {
-      const float ratio = c_prev / c;
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc[i][j][r] *= ratio;
-    }
-    Core::template gemm<LAYOUT, VEC>(p, bidx, m0, n0, acc, smem);
-    c_prev = c;
-    any = true;
-  }
-
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-  const bool single = p.groups == 1;
-  const NoiseSrc nz = p.noise.resolved();
-  const float scale = any ? c_prev * (single ? p.out_scale : 1.f) : 0.f;
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int64_t n = n0 + acc_col(wn, j, lane);
-      if (n >= p.N) continue;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t m = m0 + acc_row(wm, i, lane, r);
-        if (m >= p.M) continue;
-        float v = acc[i][j][r] * scale;
-        if (single) {
-          if (nz.on()) v += p.noise_scale * nz.at(m * p.N + n);
-          store_from_f32(p.out, m * p.ldo + n, p.out_dtype, v);
-        } else {
-          p.group_out[(int64_t(g) * p.M + m) * p.N + n] = v;
-        }
-      }
-    }
 }
 
 // out = out_scale * sum_g group_out[g] + noise_scale * noise, fixed order in g.
@@ -305,7 +204,9 @@ Plan make_plan(int64_t B, int64_t K, int64_t M, int64_t N, int cus, int flags, i
   const size_t after_partials = pl.off_partials + align_up(sizeof(float) * size_t(B) * per_sample);
   pl.off_factors = after_partials;
   pl.off_group = pl.off_factors + align_up(sizeof(float) * size_t(B));
-  const int max_groups = pl.groups > pl.sp.sum_groups ? pl.groups : pl.sp.sum_groups;
+  int max_groups = pl.groups;
+  if (pl.sp.sum.groups > max_groups) max_groups = pl.sp.sum.groups;
+  if (pl.sp.any.groups > max_groups) max_groups = pl.sp.any.groups;
   pl.total_two_pass =
       pl.off_group + (max_groups > 1 ? align_up(sizeof(float) * size_t(max_groups) * M * N) : 0);
   const GroupPlan gp = group_plan(B, pl.tiles, 2 * cus);
@@ -344,6 +245,12 @@ Plan cached_plan(int64_t B, int64_t K, int64_t M, int64_t N, int cus, int flags,
                    [&] { return make_plan(B, K, M, N, cus, flags, lda, ldb); });
 }
 
+// A plan's workspace with the partial tiles of the split Gram norm behind it.
+size_t gram_workspace(const Plan& pl, int64_t B) {
+  return align_up(pl.total) + size_t(kGramPartBytes) * size_t(B) * size_t(pl.sp.gram_per_sample) *
+                                  size_t(pl.sp.split_gram);
+}
+
 // Workspace of the fp32 schedule: partials [B, per_sample], factors [B], group
 // partials [splits, M, N].
 struct F32Layout {
@@ -379,39 +286,19 @@ F32Layout f32_layout(int64_t B, int64_t K, int64_t M, int64_t N, int layout, int
   });
 }
 
-template <class Core, int LAYOUT, bool VEC>
-hipError_t launch_passes(const Args& a, const Plan& pl, bool noclip, hipStream_t s) {
-  const dim3 block(NT);
-  if (!noclip) {
-    hipLaunchKernelGGL((wgrad_norm_kernel<Core, LAYOUT, VEC>), dim3(pl.tiles, a.B), block,
-                       Core::SMEM, s, a);
-  }
-  launch_factors(a, pl.tiles, noclip, s);
-  hipLaunchKernelGGL((wgrad_sum_kernel<Core, LAYOUT, VEC>), dim3(pl.tiles, pl.groups), block,
-                     Core::SMEM, s, a);
-  if (pl.groups > 1) launch_finalize(a, s);
-  return hipGetLastError();
-}
-
-template <class Core>
-hipError_t dispatch_layout(int layout, bool vec, const Args& a, const Plan& pl, bool noclip,
-                           hipStream_t s) {
-  if (layout == FDP_LAYOUT_TN) {
-    return vec ? launch_passes<Core, FDP_LAYOUT_TN, true>(a, pl, noclip, s)
-               : launch_passes<Core, FDP_LAYOUT_TN, false>(a, pl, noclip, s);
-  }
-  return vec ? launch_passes<Core, FDP_LAYOUT_NN, true>(a, pl, noclip, s)
-             : launch_passes<Core, FDP_LAYOUT_NN, false>(a, pl, noclip, s);
-}
-
-// Streamed two-pass schedule for 16-bit TN operands with aligned rows: Gram
-// (or direct) norms, factors, then one clipped-sum contraction per output tile.
+// Two-pass schedule of 16-bit operands: norms (Gram form, or from the products),
+// factors, then one clipped-sum contraction per output tile.  dma: the operands
+// can be read by the LDS-DMA core as they are, else they go through registers
+// (gram_part: buffer of the split Gram norm, if the plan has one and it fits).
 template <class DT>
-hipError_t launch_stream(Args a, const Plan& pl, bool noclip, hipStream_t s) {
-  const dim3 block(NT);
-  int per_sample = pl.tiles;
+hipError_t launch_two_pass(Args a, const Plan& pl, int layout, bool dma, float* gram_part,
+                           bool noclip, hipStream_t s) {
+  constexpr bool bf = DT::code == FDP_BF16;
+  int per_sample = pl.sp.norm.tiles();
+  const TilePlan& sum = dma && layout == FDP_LAYOUT_TN ? pl.sp.sum : pl.sp.any;
+  hipError_t e = hipSuccess;
   if (!noclip) {
-    if (pl.sp.gram) {
+    if (dma && layout == FDP_LAYOUT_TN && pl.sp.gram) {
       GramArgs g{};
       g.a = static_cast<const uint16_t*>(a.a);
       g.b = static_cast<const uint16_t*>(a.b);
@@ -428,26 +315,36 @@ hipError_t launch_stream(Args a, const Plan& pl, bool noclip, hipStream_t s) {
       g.items = a.B * g.per_sample;
       g.partials = a.partials;
       per_sample = g.per_sample;
-      const hipError_t e = DT::code == FDP_BF16 ? launch_gram_norm_bf16(g, s) : launch_gram_norm_f16(g, s);
-      if (e != hipSuccess) return e;
+      e = bf ? launch_gram_norm_bf16(g, s) : launch_gram_norm_f16(g, s);
+    } else if (dma) {
+      e = bf ? launch_prod_norm_bf16(a, pl.sp, layout, s) : launch_prod_norm_f16(a, pl.sp, layout, s);
     } else {
-      hipLaunchKernelGGL((wgrad_norm_kernel<Core16<DT>, FDP_LAYOUT_TN, true>), dim3(pl.tiles, a.B),
-                         block, Core16<DT>::SMEM, s, a);
+      StagedPass pass = kStagedNorm;
+      Args n = a;
+      if (layout == FDP_LAYOUT_TN && gram_part != nullptr) {
+        pass = kStagedGram;
+        n.group_out = gram_part;
+        per_sample = pl.sp.gram_per_sample;
+      }
+      e = bf ? launch_staged_bf16(n, pl.sp, layout, pass, s)
+             : launch_staged_f16(n, pl.sp, layout, pass, s);
     }
+    if (e != hipSuccess) return e;
   }
-  // The clipped-sum kernel forms the factors from the partials itself (saving
+  // The clipped-sum kernels form the factors from the partials themselves (saving
   // a launch between the passes) unless the call has no clipping or its
-  // sample groups are larger than it stages.
+  // sample groups are larger than they stage.
   a.fac_parts = 0;
-  if (!noclip && pl.sp.sum_spg <= kSumFacMax) {
-    a.fac_parts = per_sample;
-  } else {
-    launch_factors(a, per_sample, noclip, s);
-  }
-  const hipError_t e = DT::code == FDP_BF16 ? launch_clipsum_bf16(a, pl.sp, s) : launch_clipsum_f16(a, pl.sp, s);
+  if (!noclip && sum.spg <= kSumFacMax) a.fac_parts = per_sample;
+  else launch_factors(a, per_sample, noclip, s);
+  if (dma)
+    e = bf ? launch_clipsum_bf16(a, pl.sp, layout, s) : launch_clipsum_f16(a, pl.sp, layout, s);
+  else
+    e = bf ? launch_staged_bf16(a, pl.sp, layout, kStagedSum, s)
+           : launch_staged_f16(a, pl.sp, layout, kStagedSum, s);
   if (e != hipSuccess) return e;
-  if (pl.sp.sum_groups > 1) {
-    a.groups = pl.sp.sum_groups;
+  if (sum.groups > 1) {
+    a.groups = sum.groups;
     launch_finalize(a, s);
   }
   return hipGetLastError();
@@ -469,6 +366,8 @@ extern "C" int fdp_wgrad_clip_workspace_size(int64_t B, int64_t K, int64_t M, in
       const size_t t = f32_layout(B, K, M, N, layout, cus, pl.groups, false).total;
       if (t > *bytes) *bytes = t;
     }
+  } else if (pl.sp.split_gram > 0) {
+    *bytes = gram_workspace(pl, B);
   }
   return FDP_OK;
 }
@@ -695,34 +594,37 @@ int wgrad_clip_impl(const void* a, const void* b, int64_t B, int64_t K, int64_t 
   }
 
   hipError_t e;
-  // the streamed kernels address a sample's operands through 32-bit buffer
-  // records; larger samples take the generic schedule (64-bit addressing)
-  if (layout == FDP_LAYOUT_TN && vec && dtype != FDP_F32 && K > 0 && fits_record(K, lda) &&
-      fits_record(K, ldb)) {
-    args.group_out = pl.sp.sum_groups > 1 ? reinterpret_cast<float*>(ws + pl.off_group) : nullptr;
-    e = dtype == FDP_BF16 ? launch_stream<BF16>(args, pl, noclip, s)
-                          : launch_stream<F16>(args, pl, noclip, s);
+  if (dtype != FDP_F32) {
+    // The LDS-DMA kernels read 16-byte aligned rows through 32-bit buffer
+    // records (larger samples are addressed with 64 bits), and k-contiguous
+    // rows (NN) in whole k-tiles only.
+    const bool tn = layout == FDP_LAYOUT_TN;
+    const bool dma = vec && K > 0 && fits_record(tn ? K : M, lda) && fits_record(K, ldb) &&
+                     (tn || K % SumGeomNN::BK == 0);
+    if (!(tn && dma)) args.bias_op = 0;  // the caller forms the bias
+    args.group_out = reinterpret_cast<float*>(ws + pl.off_group);
+    // the split Gram norm's partial tiles follow the rest of the workspace; in a
+    // smaller one the norms come from the products
+    float* gram_part = nullptr;
+    if (pl.sp.split_gram > 0 && gram_workspace(pl, B) <= workspace_bytes)
+      gram_part = reinterpret_cast<float*>(ws + align_up(pl.total));
+    e = dtype == FDP_BF16 ? launch_two_pass<BF16>(args, pl, layout, dma, gram_part, noclip, s)
+                          : launch_two_pass<F16>(args, pl, layout, dma, gram_part, noclip, s);
     if (e != hipSuccess) return FDP_ERR_HIP;
-    if (bias_done != nullptr) *bias_done = bias != nullptr;
+    if (bias_done != nullptr) *bias_done = bias != nullptr && args.bias_op != 0;
     return FDP_OK;
   }
-  args.bias_op = 0;  // the generic schedule: the caller forms the bias
-  if (dtype == FDP_F32) {
-    // the plan that the workspace query sized, or, in a smaller workspace, the
-    // one that fits the least accepted size
-    const F32Layout fl = f32_layout(B, K, M, N, layout, cus, pl0.groups, false);
-    const F32Layout f = fl.total <= workspace_bytes
-                            ? fl
-                            : f32_layout(B, K, M, N, layout, cus, pl0.groups, true);
-    args.partials = reinterpret_cast<float*>(ws + f.off_partials);
-    args.factors = reinterpret_cast<float*>(ws + f.off_factors);
-    args.group_out = reinterpret_cast<float*>(ws + f.off_group);
-    e = launch_f32(args, f.plan, layout, noclip, s);
-  } else if (dtype == FDP_BF16) {
-    e = dispatch_layout<Core16<BF16>>(layout, vec, args, pl, noclip, s);
-  } else {
-    e = dispatch_layout<Core16<F16>>(layout, vec, args, pl, noclip, s);
-  }
+  // fp32: the plan that the workspace query sized, or, in a smaller workspace,
+  // the one that fits the least accepted size (the caller forms the bias)
+  const F32Layout fl = f32_layout(B, K, M, N, layout, cus, pl0.groups, false);
+  const F32Layout f = fl.total <= workspace_bytes
+                          ? fl
+                          : f32_layout(B, K, M, N, layout, cus, pl0.groups, true);
+  args.bias_op = 0;
+  args.partials = reinterpret_cast<float*>(ws + f.off_partials);
+  args.factors = reinterpret_cast<float*>(ws + f.off_factors);
+  args.group_out = reinterpret_cast<float*>(ws + f.off_group);
+  e = launch_f32(args, f.plan, layout, noclip, s);
   return e == hipSuccess ? FDP_OK : FDP_ERR_HIP;
 }
 
@@ -763,7 +665,7 @@ int bias_layout(int64_t B, int64_t K, int64_t M, int64_t N, int dtype, int wflag
   const int gm = static_cast<int>((M + BM - 1) / BM), gn = static_cast<int>((N + BN - 1) / BN);
   const StreamPlan sp = stream_plan(B, K, M, N, num_cus());
   const int64_t P_group = bias_op == 1 ? gn : gm, P_stream = stream_bias_P(sp, bias_op);
-  const int64_t tiles_group = int64_t(gm) * gn, tiles_stream = int64_t(sp.sum_tiles_m) * sp.sum_tiles_n;
+  const int64_t tiles_group = int64_t(gm) * gn, tiles_stream = sp.sum.tiles();
   const int64_t P = P_group > P_stream ? P_group : P_stream;
   const int64_t tiles = tiles_group > tiles_stream ? tiles_group : tiles_stream;
   const int64_t len = bias_op == 1 ? M : N;

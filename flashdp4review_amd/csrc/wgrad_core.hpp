@@ -83,174 +83,6 @@ struct Args {
   float* bias_factors;    // optional [B]: c'_b
 };
 
-// ------------------------------------------------------------------ 16-bit
-// LDS tile: [128 rows][64 k] of 16-bit values, 128 bytes per row, in 8 chunks of
-// 16 bytes whose position is XOR-swizzled by the row index.
-__device__ __forceinline__ int lds16_off(int row, int chunk) {
-  return row * 128 + ((chunk ^ ((row ^ (row >> 3)) & 7)) << 4);
-}
-
-template <class DT>
-struct Core16 {
-  using dtype = DT;
-  static constexpr int BK = 64;
-  static constexpr int TILE_BYTES = 128 * 128;  // one operand tile
-  static constexpr int SMEM = 4 * TILE_BYTES;   // 2 operands x 2 buffers
-  using Frag = uint4;
-
-  // Operand stored [K, R] with R contiguous (row stride ld).  Thread t loads
-  // rows k0+4*(t>>4)+i (i<4), columns r0+8*(t&15)..+7.
-  template <bool VEC>
-  __device__ static inline void load_kr(const uint16_t* src, int64_t ld, int64_t K, int64_t R,
-                                        int64_t k0, int64_t r0, uint4 (&reg)[4]) {
-    const int t = threadIdx.x;
-    const int64_t r = r0 + (t & 15) * 8;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int64_t k = k0 + (t >> 4) * 4 + i;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (k < K) {
-        const uint16_t* p = src + k * ld + r;
-        if (VEC && r + 8 <= R) {
-          v = *reinterpret_cast<const uint4*>(p);
-        } else {
-          uint16_t e[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) e[j] = (r + j < R) ? p[j] : uint16_t(0);
-          v.x = e[0] | (uint32_t(e[1]) << 16);
-          v.y = e[2] | (uint32_t(e[3]) << 16);
-          v.z = e[4] | (uint32_t(e[5]) << 16);
-          v.w = e[6] | (uint32_t(e[7]) << 16);
-        }
-      }
-      reg[i] = v;
-    }
-  }
-  // Transpose the 4(k) x 8(r) register block into 8 rows of 4 k-values.
-  __device__ static inline void store_kr(char* lds, const uint4 (&reg)[4]) {
-    const int t = threadIdx.x;
-    const int rc = t & 15, kq = t >> 4;
-    const uint32_t w0[4] = {reg[0].x, reg[0].y, reg[0].z, reg[0].w};
-    const uint32_t w1[4] = {reg[1].x, reg[1].y, reg[1].z, reg[1].w};
-    const uint32_t w2[4] = {reg[2].x, reg[2].y, reg[2].z, reg[2].w};
-    const uint32_t w3[4] = {reg[3].x, reg[3].y, reg[3].z, reg[3].w};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
-      const uint32_t lo = __builtin_amdgcn_perm(w1[j >> 1], w0[j >> 1], sel);
-      const uint32_t hi = __builtin_amdgcn_perm(w3[j >> 1], w2[j >> 1], sel);
-      const int row = rc * 8 + j;
-      *reinterpret_cast<uint2*>(lds + lds16_off(row, kq >> 1) + ((kq & 1) << 3)) =
-          make_uint2(lo, hi);
-    }
-  }
-  // Operand stored [R, K] with K contiguous: 16-byte chunks go straight to LDS.
-  template <bool VEC>
-  __device__ static inline void load_rk(const uint16_t* src, int64_t ld, int64_t K, int64_t R,
-                                        int64_t k0, int64_t r0, uint4 (&reg)[4]) {
-    const int t = threadIdx.x;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = t + NT * i;
-      const int64_t r = r0 + (c >> 3);
-      const int64_t k = k0 + (c & 7) * 8;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (r < R) {
-        const uint16_t* p = src + r * ld + k;
-        if (VEC && k + 8 <= K) {
-          v = *reinterpret_cast<const uint4*>(p);
-        } else {
-          uint16_t e[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) e[j] = (k + j < K) ? p[j] : uint16_t(0);
-          v.x = e[0] | (uint32_t(e[1]) << 16);
-          v.y = e[2] | (uint32_t(e[3]) << 16);
-          v.z = e[4] | (uint32_t(e[5]) << 16);
-          v.w = e[6] | (uint32_t(e[7]) << 16);
-        }
-      }
-      reg[i] = v;
-    }
-  }
-  __device__ static inline void store_rk(char* lds, const uint4 (&reg)[4]) {
-    const int t = threadIdx.x;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = t + NT * i;
-      *reinterpret_cast<uint4*>(lds + lds16_off(c >> 3, c & 7)) = reg[i];
-    }
-  }
-
-  __device__ static inline f32x16 mfma(uint4 a, uint4 b, f32x16 c) {
-    if constexpr (DT::code == FDP_BF16) {
-      return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
-                                                     __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-    } else {
-      return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
-                                                    __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-    }
-  }
-  // One BK=64 k-tile of the wave's 64x64 sub-tile.
-  __device__ static inline void mma(const char* As, const char* Bs, f32x16 (&acc)[2][2], int wm,
-                                    int wn, int lane) {
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const int chunk = ks * 2 + (lane >> 5);
-      const int rr = lane & 31;
-      const uint4 a0 = *reinterpret_cast<const uint4*>(As + lds16_off(wm + rr, chunk));
-      const uint4 a1 = *reinterpret_cast<const uint4*>(As + lds16_off(wm + 32 + rr, chunk));
-      const uint4 b0 = *reinterpret_cast<const uint4*>(Bs + lds16_off(wn + rr, chunk));
-      const uint4 b1 = *reinterpret_cast<const uint4*>(Bs + lds16_off(wn + 32 + rr, chunk));
-      acc[0][0] = mfma(a0, b0, acc[0][0]);
-      acc[0][1] = mfma(a0, b1, acc[0][1]);
-      acc[1][0] = mfma(a1, b0, acc[1][0]);
-      acc[1][1] = mfma(a1, b1, acc[1][1]);
-    }
-  }
-
-  // acc += tile (m0, n0) of G_b over the whole contraction axis.
-  template <int LAYOUT, bool VEC>
-  __device__ static void gemm(const Args& p, int64_t bidx, int64_t m0, int64_t n0,
-                              f32x16 (&acc)[2][2], char* smem) {
-    const uint16_t* A = static_cast<const uint16_t*>(p.a) + bidx * p.sab;
-    const uint16_t* Bm = static_cast<const uint16_t*>(p.b) + bidx * p.sbb;
-    // Buffer c holds the A tile at smem + 2c*TILE_BYTES and the B tile right after.
-#define FDP_AS(c) (smem + (c) * (2 * TILE_BYTES))
-#define FDP_BS(c) (smem + (c) * (2 * TILE_BYTES) + TILE_BYTES)
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-    const int nk = static_cast<int>((p.K + BK - 1) / BK);
-    uint4 ra[4], rb[4];
-    if (LAYOUT == FDP_LAYOUT_TN) load_kr<VEC>(A, p.lda, p.K, p.M, 0, m0, ra);
-    else load_rk<VEC>(A, p.lda, p.K, p.M, 0, m0, ra);
-    load_kr<VEC>(Bm, p.ldb, p.K, p.N, 0, n0, rb);
-    if (LAYOUT == FDP_LAYOUT_TN) store_kr(FDP_AS(0), ra);
-    else store_rk(FDP_AS(0), ra);
-    store_kr(FDP_BS(0), rb);
-    __syncthreads();
-    for (int kt = 0; kt < nk; ++kt) {
-      const int cur = kt & 1;
-      const bool more = kt + 1 < nk;
-      if (more) {
-        const int64_t k0 = int64_t(kt + 1) * BK;
-        if (LAYOUT == FDP_LAYOUT_TN) load_kr<VEC>(A, p.lda, p.K, p.M, k0, m0, ra);
-        else load_rk<VEC>(A, p.lda, p.K, p.M, k0, m0, ra);
-        load_kr<VEC>(Bm, p.ldb, p.K, p.N, k0, n0, rb);
-      }
-      mma(FDP_AS(cur), FDP_BS(cur), acc, wm, wn, lane);
-      if (more) {
-        if (LAYOUT == FDP_LAYOUT_TN) store_kr(FDP_AS(cur ^ 1), ra);
-        else store_rk(FDP_AS(cur ^ 1), ra);
-        store_kr(FDP_BS(cur ^ 1), rb);
-      }
-      __syncthreads();
-    }
-  }
-};
-
-#undef FDP_AS
-#undef FDP_BS
-
 __device__ __forceinline__ void zero(f32x16 (&acc)[2][2]) {
 #pragma unroll
   for (int i = 0; i < 2; ++i)

@@ -304,24 +304,112 @@ __device__ inline void store_half(const Args& p, int64_t m0, int64_t n0, int h,
   __syncthreads();
 }
 
+template <class G>
+__device__ __forceinline__ void zero_blocks(f32x16 (&acc)[G::FI][G::FJ]) {
+#pragma unroll
+  for (int i = 0; i < G::FI; ++i)
+#pragma unroll
+    for (int j = 0; j < G::FJ; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+}
+
+// This wave's sum of squares of its blocks of a tile (every lane), without what
+// lies past M and N (values of the next row or sample, or an infinite value
+// times a padding zero).
+template <class G>
+__device__ __forceinline__ float masked_squares(const Args& p, int64_t m0, int64_t n0,
+                                                const f32x16 (&acc)[G::FI][G::FJ]) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wm = (wave / G::WGN) * G::WM, wn = (wave % G::WGN) * G::WN;
+  float s = 0.f;
+  if (p.M - m0 >= G::BM && p.N - n0 >= G::BN) {
+#pragma unroll
+    for (int i = 0; i < G::FI; ++i)
+#pragma unroll
+      for (int j = 0; j < G::FJ; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s += acc[i][j][r] * acc[i][j][r];
+  } else {
+    const int ml = static_cast<int>(p.M - m0 < G::BM ? p.M - m0 : G::BM);
+    const int nl = static_cast<int>(p.N - n0 < G::BN ? p.N - n0 : G::BN);
+#pragma unroll
+    for (int i = 0; i < G::FI; ++i)
+#pragma unroll
+      for (int j = 0; j < G::FJ; ++j) {
+        const bool col = acc_col(wn, j, lane) < nl;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          s += col && acc_row(wm, i, lane, r) < ml ? acc[i][j][r] * acc[i][j][r] : 0.f;
+      }
+  }
+  return wave_sum(s);
+}
+
+// Samples per group whose clip factors a clipped-sum kernel forms itself
+// (more: wgrad_factor_kernel forms them before it).
+constexpr int kSumFacMax = 256;
+
+// The clip factors of samples [b0, b0 + nsamp) into cfac: wave w takes samples
+// w, w + 4, ... and sums each one's partials lane-strided, then across the wave
+// (the order of wgrad_factor_kernel); the workgroup of tile 0 reports them.
+__device__ inline void group_factors(const Args& p, int64_t b0, int nsamp, int tile, float* cfac) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  float C = p.C, clamp = p.clamp;
+  if (p.clip_args_dev != nullptr) {
+    C = p.clip_args_dev[0];
+    clamp = p.clip_args_dev[1];
+  }
+  for (int j = wave; j < nsamp; j += NT / kWave) {
+    const float* part = p.partials + (b0 + j) * p.fac_parts;
+    float s = 0.f;
+    for (int t = lane; t < p.fac_parts; t += kWave) s += part[t];
+    s = wave_sum(s);
+    const float n = sqrtf(s < 0.f ? 0.f : s);  // (a Gram sum may round below zero)
+    if (lane == 0) {
+      const float c = clip_factor(n, C, clamp);
+      cfac[j] = c;
+      if (tile == 0) {
+        if (p.norms_out) p.norms_out[b0 + j] = n;
+        if (p.factors_out) p.factors_out[b0 + j] = c;
+      }
+    }
+  }
+}
+
+// A contributing sample of factor c != 0 starts: the accumulator is rescaled to
+// hold sum c_j G_j / c.
+template <class G>
+__device__ __forceinline__ void start_sample(float c, float& c_prev, bool& any,
+                                             f32x16 (&acc)[G::FI][G::FJ]) {
+  if (any) {
+    const float ratio = c_prev / c;
+#pragma unroll
+    for (int i = 0; i < G::FI; ++i)
+#pragma unroll
+      for (int j = 0; j < G::FJ; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] *= ratio;
+  }
+  c_prev = c;
+  any = true;
+}
+
 // Grid: tiles x groups workgroups (XCD-aware numbering; group-major).  Group g
 // sums samples [g*spg, min(B, (g+1)*spg)) of one output tile.
 // BOP 1 / 2: also the column sums and squares of operand a / b for its bias
 // (bias_finish, run by bias_finish_kernel after this kernel): taken from the
 // fragments of every sample, also of a sample whose clip factor is zero
 // (its fragments are then read for the bias only).
-// Samples per group whose clip factors the clipped-sum kernel forms itself
-// (more: wgrad_factor_kernel forms them before it).
-constexpr int kSumFacMax = 256;
-
 template <class DT, class G, int S, int BOP = 0>
 __global__ __launch_bounds__(NT, 2) void clipsum_kernel(Args p) {
   static_assert(S >= 2 && S <= 4, "ring depth");
-  static_assert(S * G::STAGE >= G::WM * G::BN * 4, "output staging reuses the ring");
+  // (the output staging reuses the ring)
+  constexpr int kRing = S * G::STAGE > G::WM * G::BN * 4 ? S * G::STAGE : G::WM * G::BN * 4;
   constexpr int BW = BOP == 1 ? G::BM : G::BN;      // the tile's extent along the bias axis
   constexpr int NF = (BOP == 1 ? G::FI : G::FJ) / 2;  // bias fragments summed per wave
   static_assert(BOP == 0 || NF >= 1, "two waves share each row (column) of fragments");
-  __shared__ __attribute__((aligned(16))) char ring[S * G::STAGE];
+  __shared__ __attribute__((aligned(16))) char ring[kRing];
   __shared__ float bcol[BOP != 0 ? BW : 1];
   __shared__ float bred[NT / kWave];
   __shared__ float cfac[kSumFacMax];  // the group's clip factors (fac_parts > 0)
@@ -356,26 +444,21 @@ __global__ __launch_bounds__(NT, 2) void clipsum_kernel(Args p) {
   fo.init(wm, wn);
   dma::Job<G> job;
   int iu = 0, ik = 0;
-  if (nq > 0) job.init(pa + b0 * p.sab, p.lda, pb + b0 * p.sbb, p.ldb, p.K, m0, n0);
+  if (nq > 0) job.init(pa + b0 * p.sab, p.lda, pb + b0 * p.sbb, p.ldb, p.K, m0, n0, p.M);
   auto issue_next = [&](FDP_LDS char* stage) {
     job.issue(stage, ik);
     if (++ik == nk) {
       ik = 0;
       if (++iu < nsamp) {
         const int64_t b = b0 + iu;
-        job.retarget(pa + b * p.sab, p.lda, pb + b * p.sbb, p.ldb, p.K);
+        job.retarget(pa + b * p.sab, p.lda, pb + b * p.sbb, p.ldb, p.K, p.M);
       }
     }
   };
   auto stage = [&](int s) { return (FDP_LDS char*)ring + s * G::STAGE; };
 
   f32x16 acc[G::FI][G::FJ];
-#pragma unroll
-  for (int i = 0; i < G::FI; ++i)
-#pragma unroll
-    for (int j = 0; j < G::FJ; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  zero_blocks<G>(acc);
   float c_prev = 0.f;
   bool any = false, live = false;
   int cu = 0, ck = 0;
@@ -384,32 +467,9 @@ __global__ __launch_bounds__(NT, 2) void clipsum_kernel(Args p) {
 #pragma unroll
   for (int s = 0; s < S - 1; ++s)
     if (s < nq) issue_next(stage(s));
-  if (p.fac_parts > 0) {
-    // the clip factors of the group's samples, while the first stages load:
-    // wave w takes samples w, w + 4, ... and sums each one's partials
-    // lane-strided, then across the wave (the order of wgrad_factor_kernel);
-    // the workgroup of tile 0 reports them.  (Waiting for these loads also
-    // waits for the stages issued before them.)
-    float C = p.C, clamp = p.clamp;
-    if (p.clip_args_dev != nullptr) {
-      C = p.clip_args_dev[0];
-      clamp = p.clip_args_dev[1];
-    }
-    for (int j = wave; j < nsamp; j += NT / kWave) {
-      const float* part = p.partials + (b0 + j) * p.fac_parts;
-      float s = 0.f;
-      for (int t = lane; t < p.fac_parts; t += kWave) s += part[t];
-      const float n = sqrtf(wave_sum(s));
-      if (lane == 0) {
-        const float c = clip_factor(n, C, clamp);
-        cfac[j] = c;
-        if (tile == 0) {
-          if (p.norms_out) p.norms_out[b0 + j] = n;
-          if (p.factors_out) p.factors_out[b0 + j] = c;
-        }
-      }
-    }
-  }
+  // the clip factors of the group's samples, while the first stages load
+  // (waiting for these loads also waits for the stages issued before them)
+  if (p.fac_parts > 0) group_factors(p, b0, nsamp, tile, cfac);
   for (int base = 0; base < nq; base += S) {
 #pragma unroll
     for (int s = 0; s < S; ++s) {
@@ -419,22 +479,10 @@ __global__ __launch_bounds__(NT, 2) void clipsum_kernel(Args p) {
         dma::wait_tiles<G::LOADS>(ahead < S - 2 ? ahead : S - 2);
         dma::barrier();
         if (q + S - 1 < nq) issue_next(stage((s + S - 1) % S));
-        if (ck == 0) {  // sample b0 + cu starts: rescale to its factor
+        if (ck == 0) {  // sample b0 + cu starts
           const float c = p.fac_parts > 0 ? cfac[cu] : p.factors[b0 + cu];
           live = c != 0.f;  // a zero factor contributes exactly nothing
-          if (live) {
-            if (any) {
-              const float ratio = c_prev / c;
-#pragma unroll
-              for (int i = 0; i < G::FI; ++i)
-#pragma unroll
-                for (int j = 0; j < G::FJ; ++j)
-#pragma unroll
-                  for (int r = 0; r < 16; ++r) acc[i][j][r] *= ratio;
-            }
-            c_prev = c;
-            any = true;
-          }
+          if (live) start_sample<G>(c, c_prev, any, acc);
         }
         if (live) dma::compute_stage<DT, G>(stage(s), fo, acc);
         if constexpr (BOP != 0) {
@@ -472,38 +520,125 @@ __global__ __launch_bounds__(NT, 2) void clipsum_kernel(Args p) {
   }
 }
 
+// Per-(tile, sample) squares of the products, where the Gram form is not
+// cheaper or not possible: the same tiles and ring as the clipped sum, so both
+// passes run at its rate.  Grid: tiles x B workgroups, sample-major.
+template <class DT, class G, int S>
+__global__ __launch_bounds__(NT, 2) void prod_norm_kernel(Args p) {
+  __shared__ __attribute__((aligned(16))) char ring[S * G::STAGE];
+  __shared__ float red[NT / kWave];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int tiles = p.tiles_m * p.tiles_n;
+  const int64_t units = p.B * tiles;
+  for (int64_t u = logical_wg(blockIdx.x, gridDim.x); u < units; u += gridDim.x) {
+    const int64_t b = u / tiles;
+    const int tile = static_cast<int>(u - b * tiles);
+    int64_t m0, n0;
+    tile_coords_g<G>(p, tile, m0, n0);
+    dma::FragOffsets<G> fo;
+    fo.init((wave / G::WGN) * G::WM, (wave % G::WGN) * G::WN);
+    dma::Job<G> job;
+    job.init(static_cast<const uint16_t*>(p.a) + b * p.sab, p.lda,
+             static_cast<const uint16_t*>(p.b) + b * p.sbb, p.ldb, p.K, m0, n0, p.M);
+    dma::Stages st{};
+#pragma unroll
+    for (int s = 0; s < S; ++s) st.s[s] = (FDP_LDS char*)ring + s * G::STAGE;
+    f32x16 acc[G::FI][G::FJ];
+    zero_blocks<G>(acc);
+    dma::gemm<DT, G, S>(job, static_cast<int>((p.K + G::BK - 1) / G::BK), fo, st, acc);
+    const float s = masked_squares<G>(p, m0, n0, acc);
+    if (lane == 0) red[wave] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) p.partials[u] = (red[0] + red[1]) + (red[2] + red[3]);
+    __syncthreads();
+  }
+}
+
 // ------------------------------------------------------------------ host
 // Geometry of the clipped-sum pass: 128 x 256 output tiles (each wave 64 x 128,
 // 2 x 4 MFMA blocks), 32-deep k-tiles in a 3-stage ring (72 KB, two
 // workgroups per CU).
 using SumGeom = dma::Geom<128, 256, 32>;
+using SumGeomNN = dma::Geom<128, 256, 32, 2, 2, true, false>;  // a: [M, K], k contiguous
 constexpr int kSumStages = 3;
 
+using SmallGeom = dma::Geom<128, 128, 32>;    // layers of few 128 x 256 tiles
+using SmallGeomNN = dma::Geom<128, 128, 32, 2, 2, true, false>;
+
+// Output tiles of one pass and the sample groups that share them.
+struct TilePlan {
+  int tiles_m, tiles_n, groups, spg;
+  int tiles() const { return tiles_m * tiles_n; }
+  void set(Args& a) const {
+    a.tiles_m = tiles_m;
+    a.tiles_n = tiles_n;
+    a.groups = groups;
+    a.spg = spg;
+  }
+};
+
 struct StreamPlan {
-  int sum_tiles_m, sum_tiles_n, sum_groups, sum_spg;
+  TilePlan sum;   // clipped sum on 128 x 256 tiles
+  TilePlan any;   // the clipped sum of operands other than aligned TN ones
+  bool any_small;   // `any` is on 128 x 128 tiles
+  TilePlan norm;  // squares of the products (groups unused)
+  bool norm_small;
   int gram_nt, gram_per_sample;
   bool gram;  // the Gram norm is used (cheaper and shape-compatible)
+  int split_gram;  // > 0: unaligned TN operands take the split Gram norm, in so many parts
 };
+
+constexpr double kGramPartBytes = 4. * kGramT * kGramT;
 
 inline StreamPlan stream_plan(int64_t B, int64_t K, int64_t M, int64_t N, int cus) {
   StreamPlan s{};
-  s.sum_tiles_m = static_cast<int>((M + SumGeom::BM - 1) / SumGeom::BM);
-  s.sum_tiles_n = static_cast<int>((N + SumGeom::BN - 1) / SumGeom::BN);
-  const int64_t tiles = int64_t(s.sum_tiles_m) * s.sum_tiles_n;
   // split the batch into groups while tiles x groups workgroups stay within
   // one wave of two per CU (a second, partial wave would cost a whole extra
   // tile time), keeping the fp32 group partials at or below B*M*N bytes
-  int64_t want = 2 * int64_t(cus) / tiles;
-  const int64_t cap = B / 4 > 1 ? B / 4 : 1;
-  if (want > cap) want = cap;
-  if (want < 1) want = 1;
-  s.sum_spg = static_cast<int>((B + want - 1) / want);
-  s.sum_groups = static_cast<int>((B + s.sum_spg - 1) / s.sum_spg);
+  auto plan = [&](int bn) {
+    TilePlan t{};
+    t.tiles_m = static_cast<int>((M + SumGeom::BM - 1) / SumGeom::BM);
+    t.tiles_n = static_cast<int>((N + bn - 1) / bn);
+    int64_t want = 2 * int64_t(cus) / t.tiles();
+    const int64_t cap = B / 4 > 1 ? B / 4 : 1;
+    if (want > cap) want = cap;
+    if (want < 1) want = 1;
+    t.spg = static_cast<int>((B + want - 1) / want);
+    t.groups = static_cast<int>((B + t.spg - 1) / t.spg);
+    return t;
+  };
+  s.sum = s.any = s.norm = plan(SumGeom::BN);
+  const TilePlan small = plan(SmallGeom::BN);
+  // a CU needs two 4-wave workgroups to run near its rate: where the 128 x 256
+  // tiles give fewer, halve them (bmm_clip of 16 x [768, 1024] x [1024, 2304], one
+  // workgroup per CU: 81 us; on 128 x 128 tiles, two: 69 us)
+  if (int64_t(s.any.tiles()) * s.any.groups < 2 * int64_t(cus) &&
+      small.tiles() * small.groups > s.any.tiles() * s.any.groups) {
+    s.any = small;
+    s.any_small = true;
+  }
+  if (int64_t(s.norm.tiles()) * B < 2 * int64_t(cus)) {
+    s.norm = small;
+    s.norm_small = true;
+  }
   s.gram_nt = static_cast<int>((K + kGramT - 1) / kGramT);
   s.gram_per_sample = s.gram_nt * (s.gram_nt + 1) / 2;
   const double direct = double(K) * M * N;
   const double gram = double(s.gram_per_sample) * kGramT * kGramT * double(M + N);
   s.gram = M % 64 == 0 && N % 64 == 0 && K > 0 && gram < direct;
+  // the split Gram norm (wgrad_staged.hpp): the longer operand's Gram tiles are
+  // contracted in parts until there are two workgroups per CU, of at least 8
+  // k-tiles each, with at most 64 MB of partial tiles
+  const double items = double(B) * s.gram_per_sample;
+  const int64_t longer = M > N ? M : N;
+  if ((M % 8 != 0 || N % 8 != 0) && K > 0 && gram < 0.8 * direct &&
+      items * kGramPartBytes <= 64e6) {
+    int64_t parts = static_cast<int64_t>(2. * cus / items);
+    if (parts * items * kGramPartBytes > 64e6)
+      parts = static_cast<int64_t>(64e6 / (items * kGramPartBytes));
+    if (parts > (longer + 511) / 512) parts = (longer + 511) / 512;
+    s.split_gram = parts < 1 ? 1 : static_cast<int>(parts);
+  }
   return s;
 }
 
@@ -514,21 +649,44 @@ hipError_t launch_gram_norm(const GramArgs& g, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <class DT, class G>
+void launch_prod_norm_geom(const Args& a, hipStream_t s) {
+  const int64_t units = a.B * a.tiles_m * a.tiles_n;
+  const dim3 grid(static_cast<unsigned>(units < (1 << 30) ? units : (1 << 30)));
+  hipLaunchKernelGGL((prod_norm_kernel<DT, G, kSumStages>), grid, dim3(NT), 0, s, a);
+}
+template <class DT>
+hipError_t launch_prod_norm(Args a, const StreamPlan& sp, int layout, hipStream_t s) {
+  sp.norm.set(a);
+  const bool tn = layout == FDP_LAYOUT_TN;
+  if (tn && sp.norm_small) launch_prod_norm_geom<DT, SmallGeom>(a, s);
+  else if (tn) launch_prod_norm_geom<DT, SumGeom>(a, s);
+  else if (sp.norm_small) launch_prod_norm_geom<DT, SmallGeomNN>(a, s);
+  else launch_prod_norm_geom<DT, SumGeomNN>(a, s);
+  return hipGetLastError();
+}
+
 // Partials per bias output of the clipped-sum pass (tiles along the other axis).
 inline int stream_bias_P(const StreamPlan& sp, int bias_op) {
-  return bias_op == 1 ? sp.sum_tiles_n : sp.sum_tiles_m;
+  return bias_op == 1 ? sp.sum.tiles_n : sp.sum.tiles_m;
 }
 
 // The clipped-sum pass; with a.bias_op, also the bias (bias_finish_kernel
 // after the pass, one workgroup per kBiasCols outputs).
 template <class DT>
-hipError_t launch_clipsum(Args a, const StreamPlan& sp, hipStream_t s) {
-  a.tiles_m = sp.sum_tiles_m;
-  a.tiles_n = sp.sum_tiles_n;
-  a.groups = sp.sum_groups;
-  a.spg = sp.sum_spg;
+hipError_t launch_clipsum(Args a, const StreamPlan& sp, int layout, hipStream_t s) {
+  (layout == FDP_LAYOUT_TN ? sp.sum : sp.any).set(a);
   const int tiles = a.tiles_m * a.tiles_n;
   const unsigned grid = static_cast<unsigned>(tiles * a.groups);
+  if (layout == FDP_LAYOUT_NN) {  // (no bias there)
+    if (sp.any_small)
+      hipLaunchKernelGGL((clipsum_kernel<DT, SmallGeomNN, kSumStages, 0>), dim3(grid), dim3(NT), 0,
+                         s, a);
+    else
+      hipLaunchKernelGGL((clipsum_kernel<DT, SumGeomNN, kSumStages, 0>), dim3(grid), dim3(NT), 0,
+                         s, a);
+    return hipGetLastError();
+  }
   if (a.bias_op == 0) {
     hipLaunchKernelGGL((clipsum_kernel<DT, SumGeom, kSumStages, 0>), dim3(grid), dim3(NT), 0, s, a);
     return hipGetLastError();
@@ -550,8 +708,10 @@ hipError_t launch_clipsum(Args a, const StreamPlan& sp, hipStream_t s) {
 // Per-dtype instantiations (wgrad_stream_{bf16,f16}.hip).
 hipError_t launch_gram_norm_bf16(const GramArgs& g, hipStream_t s);
 hipError_t launch_gram_norm_f16(const GramArgs& g, hipStream_t s);
-hipError_t launch_clipsum_bf16(const Args& a, const StreamPlan& sp, hipStream_t s);
-hipError_t launch_clipsum_f16(const Args& a, const StreamPlan& sp, hipStream_t s);
+hipError_t launch_clipsum_bf16(const Args& a, const StreamPlan& sp, int layout, hipStream_t s);
+hipError_t launch_clipsum_f16(const Args& a, const StreamPlan& sp, int layout, hipStream_t s);
+hipError_t launch_prod_norm_bf16(const Args& a, const StreamPlan& sp, int layout, hipStream_t s);
+hipError_t launch_prod_norm_f16(const Args& a, const StreamPlan& sp, int layout, hipStream_t s);
 
 }  // namespace wg
 }  // namespace fdp

@@ -8,8 +8,11 @@ namespace wg {
 hipError_t launch_gram_norm_bf16(const GramArgs& g, hipStream_t s) {
   return launch_gram_norm<BF16>(g, s);
 }
-hipError_t launch_clipsum_bf16(const Args& a, const StreamPlan& sp, hipStream_t s) {
-  return launch_clipsum<BF16>(a, sp, s);
+hipError_t launch_clipsum_bf16(const Args& a, const StreamPlan& sp, int layout, hipStream_t s) {
+  return launch_clipsum<BF16>(a, sp, layout, s);
+}
+hipError_t launch_prod_norm_bf16(const Args& a, const StreamPlan& sp, int layout, hipStream_t s) {
+  return launch_prod_norm<BF16>(a, sp, layout, s);
 }
 
 }  // namespace wg

@@ -1,0 +1,91 @@
+"""16-bit two-pass schedules beside the Gram one, at the edges of their rules
+(csrc/wgrad_staged.hpp, prod_norm_kernel and the NN clipped sum of
+csrc/wgrad_stream.hpp): rows that are not 16-byte aligned, operands narrower
+than a 16-byte chunk, a contraction that fills no k-tile, exactly one, or
+leaves a remainder; edge tiles of 128 x 256; grouped samples.
+
+Against the float64 oracle on the same rounded operands: the products are
+accumulated in fp32 and the fp32 output is not rounded, so fp32's bar holds
+(K <= 300 terms: 300 * 2^-24 = 2e-5 of the largest partial sum at worst, and
+random signs keep it below 1e-5 of the result).
+"""
+import numpy as np
+import pytest
+import torch
+
+from oracle import dp_clip as O
+from tests._tol import assert_close, assert_elementwise
+
+from flashdp4review_amd import core
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+SHAPES = [  # B, K, M, N
+    (3, 5, 3, 2),          # rows shorter than a chunk
+    (2, 33, 7, 300),       # operand a narrower than a chunk, two k-tiles
+    (4, 32, 129, 257),     # one whole k-tile, odd widths, ragged tiles
+    (3, 64, 128, 256),     # whole tiles and k-tiles (aligned)
+    (2, 96, 130, 512),     # a ragged, b whole
+    (3, 95, 261, 777),     # every edge ragged, the last k-tile too
+    (5, 31, 1, 1),
+    (16, 160, 200, 264),   # grouped samples, aligned
+    (9, 300, 131, 513),
+    # split Gram norms (TN): one and several Gram tiles a sample, ragged rows,
+    # either operand the wider one, parts of unequal length
+    (2, 128, 3001, 130),
+    (3, 130, 70, 2049),
+    (1, 257, 5003, 259),
+]
+
+
+def make(B, K, M, N, dtype, layout, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    a = torch.randn((B, K, M) if layout == "tn" else (B, M, K), generator=g)
+    b = torch.randn(B, K, N, generator=g) * (0.1 + torch.rand(B, 1, 1, generator=g))
+    return a.to(dtype).to(DEV), b.to(dtype).to(DEV)
+
+
+@pytest.mark.parametrize("layout", ["tn", "nn"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_two_pass_parity(shape, dtype, layout):
+    B, K, M, N = shape
+    a, b = make(B, K, M, N, dtype, layout)
+    _, norms_ref, _ = O.wgrad_clip(a, b, 1.0, 1.0, layout)
+    C = float(np.median(norms_ref))
+    ref, norms_ref, fac_ref = O.wgrad_clip(a, b, C, 1.0, layout)
+    out, norms, fac = core.wgrad_clip(a, b, C, 1.0, layout=layout, out_dtype=torch.float32,
+                                      two_pass=True, return_stats=True)
+    assert_close(out, ref, torch.float32, "sum")
+    assert_elementwise(norms, norms_ref, torch.float32, "norms")
+    assert_elementwise(fac, fac_ref, torch.float32, "factors")
+    # the same rows inside a wider allocation, one element off a 16-byte boundary,
+    # with infinities in what lies around them
+    def off(t):
+        w = torch.full((t.shape[0], t.shape[1] + 2, t.shape[2] + 9), float("inf"), dtype=dtype,
+                       device=DEV)
+        v = w[:, 1:-1, 1:t.shape[2] + 1]
+        v.copy_(t)
+        return v
+    o2, n2, _ = core.wgrad_clip(off(a), off(b), C, 1.0, layout=layout, out_dtype=torch.float32,
+                                two_pass=True, return_stats=True)
+    assert_close(o2, ref, torch.float32, "offset sum")
+    assert_elementwise(n2, norms_ref, torch.float32, "offset norms")
+
+
+def test_last_rows_of_an_allocation():
+    """Operands that end with their allocation's last bytes (a whole 2 MB one):
+    nothing past them is read as data."""
+    B, K, M, N = 2, 40, 131, 133
+    n = 1 << 20
+    a, b = make(B, K, M, N, torch.bfloat16, "tn", seed=3)
+    ref, _, _ = O.wgrad_clip(a, b, 1.0, 1.0, "tn")
+    bufs = [torch.empty(n, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    views = []
+    for t, w in zip((a, b), bufs):
+        v = w[n - t.numel():].view(t.shape)
+        v.copy_(t)
+        views.append(v)
+    out = core.wgrad_clip(*views, 1.0, 1.0, out_dtype=torch.float32, two_pass=True)
+    assert_close(out, ref, torch.float32)
