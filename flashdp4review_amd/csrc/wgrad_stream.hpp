@@ -22,6 +22,8 @@
 // sum pass reads the [T, M] / [T, N] operands with transposing LDS reads.
 #pragma once
 
+#include <cmath>
+
 #include "wgrad_core.hpp"
 
 namespace fdp {
@@ -594,13 +596,17 @@ inline StreamPlan stream_plan(int64_t B, int64_t K, int64_t M, int64_t N, int cu
   StreamPlan s{};
   // split the batch into groups while tiles x groups workgroups stay within
   // one wave of two per CU (a second, partial wave would cost a whole extra
-  // tile time), keeping the fp32 group partials at or below B*M*N bytes
+  // tile time), keeping the fp32 group partials at or below B*M*N bytes or, in
+  // layers so small that a workgroup would otherwise walk many short samples
+  // alone, 8 MB
   auto plan = [&](int bn) {
     TilePlan t{};
     t.tiles_m = static_cast<int>((M + SumGeom::BM - 1) / SumGeom::BM);
     t.tiles_n = static_cast<int>((N + bn - 1) / bn);
     int64_t want = 2 * int64_t(cus) / t.tiles();
-    const int64_t cap = B / 4 > 1 ? B / 4 : 1;
+    int64_t cap = static_cast<int64_t>(8e6 / (4. * double(M) * double(N)));
+    if (cap > B) cap = B;
+    if (cap < B / 4) cap = B / 4;
     if (want > cap) want = cap;
     if (want < 1) want = 1;
     t.spg = static_cast<int>((B + want - 1) / want);
@@ -629,15 +635,26 @@ inline StreamPlan stream_plan(int64_t B, int64_t K, int64_t M, int64_t N, int cu
   // the split Gram norm (wgrad_staged.hpp): the longer operand's Gram tiles are
   // contracted in parts until there are two workgroups per CU, of at least 8
   // k-tiles each, with at most 64 MB of partial tiles
-  const double items = double(B) * s.gram_per_sample;
-  const int64_t longer = M > N ? M : N;
+  const double items = double(B) * s.gram_per_sample, slots = 2. * cus;
   if ((M % 8 != 0 || N % 8 != 0) && K > 0 && gram < 0.8 * direct &&
       items * kGramPartBytes <= 64e6) {
-    int64_t parts = static_cast<int64_t>(2. * cus / items);
+    const double longer = double((M > N ? M : N) + 63) / 64, shorter = double((M > N ? N : M) + 63) / 64;
+    int64_t parts = static_cast<int64_t>(slots / items);
     if (parts * items * kGramPartBytes > 64e6)
       parts = static_cast<int64_t>(64e6 / (items * kGramPartBytes));
-    if (parts > (longer + 511) / 512) parts = (longer + 511) / 512;
-    s.split_gram = parts < 1 ? 1 : static_cast<int>(parts);
+    if (parts > longer / 8) parts = static_cast<int64_t>(longer / 8);
+    if (parts < 1) parts = 1;
+    // Estimated us, from kernel times: a 64-deep k-tile of a Gram workgroup takes
+    // 1.9 us (the join's, one workgroup per CU, 1.3, and 0.8 per part read); a
+    // 32-deep one of the products 2.5, and each round of tiles 3 more.  4 x 512,
+    // 768 -> 50257: 164 us against 404; 4 x 51, 865 -> 2561: 48 against 11.  (With a
+    // fuller Gram form than products, it lost: 9 x 362, 228 -> 4416, whole call
+    // 137 against 111 us.)
+    const double split = std::ceil(items * parts / slots) * longer / parts * 1.9 +
+                         std::ceil(items / slots) * (shorter * 1.3 + parts * 0.8) + 12.;
+    const double prod = std::ceil(double(s.norm.tiles()) * B / slots) *
+                        (static_cast<double>((K + 31) / 32) * 2.5 + 3.);
+    if (split < prod) s.split_gram = static_cast<int>(parts);
   }
   return s;
 }

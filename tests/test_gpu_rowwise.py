@@ -8,7 +8,7 @@ import torch.nn.functional as F
 from oracle import dp_clip as O
 from tests._tol import assert_close, assert_elementwise
 
-from flashdp4review_amd import core
+from flashdp4review_amd import _lib, core
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -314,3 +314,50 @@ def test_colsum_and_layernorm_in_kernel_noise():
     zb = PX.normals(1024, *key, stream=1)
     assert np.max(np.abs((w1 - w0).double().cpu().numpy() / 0.3 - zw)) < 1e-4
     assert np.max(np.abs((b1 - b0).double().cpu().numpy() / 0.3 - zb)) < 1e-4
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("H", [1, 2, 3, 6, 65, 513, 1001, 1002, 2050, 3999, 4094, 8190, 16382])
+def test_rows_of_whole_dwords(H, dtype):
+    """Rows that are no multiple of 16 bytes: LayerNorm forward and backward with
+    16-byte accesses where a row is whole dwords (its last vector is cut by the row's
+    buffer resource), element ones otherwise, from inputs one element off a 16-byte
+    boundary; nothing is written before, between or past the rows; column sums whose
+    partials are padded to items of 4 columns."""
+    B, T = 3, 9
+    n = B * T * H
+    off = 1 if dtype == torch.float32 else 2
+    x, g = randn((n + off,), dtype, 50)[off:].view(B, T, H), randn((n + off,), dtype, 51, 0.01)[off:].view(B, T, H)
+    w, b = randn((H,), dtype, 52), randn((H,), dtype, 53)
+    y, mean, rstd = core.layernorm_fwd(x, w, b, 1e-5)
+    yr, mr, rr = O.layernorm_fwd(x, w, b, 1e-5)
+    assert_close(y, yr, dtype, "y")
+    assert_elementwise(rstd.reshape(rr.shape), rr, dtype, "rstd")
+    r0 = O.layernorm_bwd_clip(g, x, w, 1e-5, C=1.0, mean=mean, rstd=rstd)
+    C = float(np.median(r0["norms_b"]))
+    ref = O.layernorm_bwd_clip(g, x, w, 1e-5, C=C, mean=mean, rstd=rstd)
+    ws = torch.empty(1 << 20, dtype=torch.uint8, device=DEV)
+    wide = torch.full((n + 64,), 7.0, dtype=dtype, device=DEV)
+    dx = wide[32:32 + n]
+    dw, db = torch.empty(H, dtype=dtype, device=DEV), torch.empty(H, dtype=dtype, device=DEV)
+    L = _lib.lib()
+    dt = _lib.dtype_code(dtype)
+    st = L.fdp_layernorm_bwd_clip(
+        g.data_ptr(), x.data_ptr(), w.data_ptr(), mean.data_ptr(), rstd.data_ptr(), B, T, H, dt, dt,
+        C, 1.0, None, 1.0 / B, None, None, 0.0, None, dx.data_ptr(), dw.data_ptr(), db.data_ptr(),
+        None, None, ws.data_ptr(), ws.numel(), _lib.stream_handle(ws.device))
+    assert st == 0
+    assert torch.all(wide[:32] == 7) and torch.all(wide[32 + n:] == 7)
+    # (x_hat of one column is rounding noise, and dx of two is: x_hat = +-1, so that
+    # dx is eps / var of its terms and fp32's 1e-7 of those is most of it)
+    if H > 2:
+        assert_close(dx.view(B, T, H), ref["dx"], dtype, "dx")
+        assert_close(dw, ref["dw"], dtype, "dgamma")
+    assert_close(db, ref["db"], dtype, "dbeta")
+    s, norms, _ = core.colsum_clip(g, None, C, 1.0, norm="frob", out_dtype=torch.float32,
+                                   return_stats=True)
+    gf = g.double().cpu().numpy()
+    nr = np.sqrt((gf ** 2).sum((1, 2)))
+    assert_elementwise(norms, nr, torch.float32, "norms")
+    assert_close(s, (np.minimum(1.0, C / (nr + 1e-10))[:, None] * gf.sum(1)).sum(0), torch.float32,
+                 "column sums")
