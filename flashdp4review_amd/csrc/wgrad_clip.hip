@@ -251,21 +251,28 @@ size_t gram_workspace(const Plan& pl, int64_t B) {
                                   size_t(pl.sp.split_gram);
 }
 
-// Workspace of the fp32 schedule: partials [B, per_sample], factors [B], group
-// partials [splits, M, N].
+// Workspace of the fp32 schedules: of the two-pass one, partials [B, per_sample],
+// factors [B], group partials [splits, M, N]; of the paired one, as in Plan.
 struct F32Layout {
   F32Plan plan;
   size_t off_partials, off_factors, off_group, total;
+  WidePlan wp;
+  size_t off_slots, off_bias_part, off_bias_sq, total_pair;
 };
+
+// Smallest share of the CUs that the paired kernel's fp32 products must fill: it
+// forms every product once, the two-pass schedule twice (or once and a Gram
+// form), so a half-filled grid breaks even.
+constexpr double kPairF32MinFill = 0.45;
 
 // Splits of the fp32 sum pass: their partials stay below one fp32 gradient per
 // sample or 32 MB, whichever is more, and below 256 MB.  lean: the plan that
 // fits a workspace of make_plan's size (old_groups group partials).
 F32Layout f32_layout(int64_t B, int64_t K, int64_t M, int64_t N, int layout, int cus,
-                     int old_groups, bool lean) {
-  using Key = std::tuple<int64_t, int64_t, int64_t, int64_t, int, int, int, bool>;
+                     int old_groups, int flags, bool lean) {
+  using Key = std::tuple<int64_t, int64_t, int64_t, int64_t, int, int, int, int, bool>;
   static host::ShapeCache<Key, F32Layout> cache;
-  return cache.get(Key{B, K, M, N, layout, cus, old_groups, lean}, [&] {
+  return cache.get(Key{B, K, M, N, layout, cus, old_groups, flags, lean}, [&] {
     F32Layout l{};
     const double mn = 4. * double(M) * double(N);
     int64_t most = old_groups;
@@ -282,6 +289,16 @@ F32Layout f32_layout(int64_t B, int64_t K, int64_t M, int64_t N, int layout, int
     l.total = l.off_group;
     if (l.plan.splits > 1)
       l.total += align_up(sizeof(float) * size_t(l.plan.splits) * size_t(M) * size_t(N));
+    if (!lean && layout == FDP_LAYOUT_TN && K > 0 && !(flags & (FDP_WGRAD_NARROW |
+        FDP_WGRAD_TWO_PASS | FDP_WGRAD_UNPAIRED | FDP_WGRAD_NOCLIP))) {
+      l.wp = wide_plan(B, K, M, N, M, N, cus, (flags & FDP_WGRAD_WIDE) ? 0.0 : kPairF32MinFill, true);
+      if (l.wp.pair != 0) {
+        l.off_slots = kWsHead + align_up(l.wp.partial_bytes);
+        l.off_bias_part = l.off_slots + align_up(l.wp.slot_bytes);
+        l.off_bias_sq = l.off_bias_part + align_up(l.wp.bias_part_bytes);
+        l.total_pair = l.off_bias_sq + l.wp.bias_sq_bytes;
+      }
+    }
     return l;
   });
 }
@@ -363,8 +380,9 @@ extern "C" int fdp_wgrad_clip_workspace_size(int64_t B, int64_t K, int64_t M, in
   *bytes = pl.total;
   if (dtype == FDP_F32) {
     for (int layout : {FDP_LAYOUT_TN, FDP_LAYOUT_NN}) {
-      const size_t t = f32_layout(B, K, M, N, layout, cus, pl.groups, false).total;
-      if (t > *bytes) *bytes = t;
+      const F32Layout l = f32_layout(B, K, M, N, layout, cus, pl.groups, flags, false);
+      if (l.total > *bytes) *bytes = l.total;
+      if (l.total_pair > *bytes) *bytes = l.total_pair;
     }
   } else if (pl.sp.split_gram > 0) {
     *bytes = gram_workspace(pl, B);
@@ -490,12 +508,9 @@ int wgrad_clip_impl(const void* a, const void* b, int64_t B, int64_t K, int64_t 
                    ldb % vel == 0 && stride_ab % vel == 0 && stride_bb % vel == 0;
 
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // Wide single pass: 16-bit TN inputs, aligned rows, two samples' products
-  // per CU (paired) or one.
-  const bool pair = pl.wp.pair != 0 && pair_records_fit(K, lda, stride_ab) &&
-                    pair_records_fit(K, ldb, stride_bb);
-  if (!noclip && (flags & FDP_WGRAD_TWO_PASS) == 0 && layout == FDP_LAYOUT_TN && vec && K > 0 &&
-      dtype != FDP_F32 && (pair || pl.wp.wgm != 0)) {
+  // The wide kernels' arguments: plan and workspace parts of the call.
+  auto wide_args = [&](const WidePlan& wp, bool pair, size_t off_partials, size_t off_slots,
+                       size_t off_bias_part, size_t off_bias_sq) {
     WideArgs w{};
     w.a = static_cast<const uint16_t*>(a);
     w.b = static_cast<const uint16_t*>(b);
@@ -507,15 +522,15 @@ int wgrad_clip_impl(const void* a, const void* b, int64_t B, int64_t K, int64_t 
     w.lda = lda;
     w.sbb = stride_bb;
     w.ldb = ldb;
-    w.tiles_m = pair ? pl.wp.pair_tiles_m : pl.wp.tiles_m;
-    w.tiles_n = pair ? pl.wp.pair_tiles_n : pl.wp.tiles_n;
-    w.tiles = pair ? pl.wp.pair_tiles : pl.wp.tiles;
-    w.nwg = pair ? pl.wp.pair_nwg : pl.wp.nwg;
-    w.partials = reinterpret_cast<float*>(ws + pl.off_wide_partials);
-    w.slots = ws + pl.off_wide_slots;
-    w.slot_blocks = pair ? pl.wp.pair_slot_blocks : pl.wp.slot_blocks;
+    w.tiles_m = pair ? wp.pair_tiles_m : wp.tiles_m;
+    w.tiles_n = pair ? wp.pair_tiles_n : wp.tiles_n;
+    w.tiles = pair ? wp.pair_tiles : wp.tiles;
+    w.nwg = pair ? wp.pair_nwg : wp.nwg;
+    w.partials = reinterpret_cast<float*>(ws + off_partials);
+    w.slots = ws + off_slots;
+    w.slot_blocks = pair ? wp.pair_slot_blocks : wp.slot_blocks;
     w.group_cnt = reinterpret_cast<unsigned*>(ws) + kGroupWord0;
-    w.tagged = reinterpret_cast<uint64_t*>(ws + pl.off_wide_partials);
+    w.tagged = reinterpret_cast<uint64_t*>(ws + off_partials);
     w.out = out;
     w.ldo = ldo;
     w.out_dtype = out_dtype;
@@ -534,10 +549,10 @@ int wgrad_clip_impl(const void* a, const void* b, int64_t B, int64_t K, int64_t 
     w.factors_out = factors;
     if (bias != nullptr) {
       w.bias_op = bias_op;
-      w.bias_part = reinterpret_cast<float*>(ws + pl.off_wide_bias_part);
-      w.bias_sq = reinterpret_cast<float*>(ws + pl.off_wide_bias_sq);
-      w.bias_tagged = reinterpret_cast<uint64_t*>(ws + pl.off_wide_bias_part);
-      w.bias_sq_tagged = reinterpret_cast<uint64_t*>(ws + pl.off_wide_bias_sq);
+      w.bias_part = reinterpret_cast<float*>(ws + off_bias_part);
+      w.bias_sq = reinterpret_cast<float*>(ws + off_bias_sq);
+      w.bias_tagged = reinterpret_cast<uint64_t*>(ws + off_bias_part);
+      w.bias_sq_tagged = reinterpret_cast<uint64_t*>(ws + off_bias_sq);
       w.bias_out = bias->out;
       w.bias_dtype = bias->out_dtype;
       w.bias_scale = bias->out_scale;
@@ -551,12 +566,24 @@ int wgrad_clip_impl(const void* a, const void* b, int64_t B, int64_t K, int64_t 
       const int oes = out_dtype == FDP_F32 ? 4 : 2;
       w.vec_out = (reinterpret_cast<uintptr_t>(out) % (4 * oes) == 0 && ldo % 4 == 0) ? 1 : 0;
     }
+    return w;
+  };
+  auto clear_head = [&] {
+    if ((flags & FDP_WGRAD_CLEAN_WORKSPACE) != 0) return;
+    const int64_t words = int64_t(kWsHead / sizeof(unsigned));
+    hipLaunchKernelGGL(clear_words_kernel<0>, dim3(static_cast<unsigned>((words + NT - 1) / NT)),
+                       dim3(NT), 0, s, reinterpret_cast<unsigned*>(ws), words);
+  };
+  // Wide single pass: 16-bit TN inputs, aligned rows, two samples' products
+  // per CU (paired) or one.
+  const bool pair = pl.wp.pair != 0 && pair_records_fit(K, lda, stride_ab) &&
+                    pair_records_fit(K, ldb, stride_bb);
+  if (!noclip && (flags & FDP_WGRAD_TWO_PASS) == 0 && layout == FDP_LAYOUT_TN && vec && K > 0 &&
+      dtype != FDP_F32 && (pair || pl.wp.wgm != 0)) {
+    const WideArgs w = wide_args(pl.wp, pair, pl.off_wide_partials, pl.off_wide_slots,
+                                 pl.off_wide_bias_part, pl.off_wide_bias_sq);
     const bool plain = (flags & FDP_WGRAD_PLAIN_LAUNCH) != 0;
-    if ((flags & FDP_WGRAD_CLEAN_WORKSPACE) == 0) {
-      const int64_t words = int64_t(kWsHead / sizeof(unsigned));
-      hipLaunchKernelGGL(clear_words_kernel<0>, dim3(static_cast<unsigned>((words + NT - 1) / NT)),
-                         dim3(NT), 0, s, reinterpret_cast<unsigned*>(ws), words);
-    }
+    clear_head();
     const int wgm = pair ? 1 : pl.wp.wgm;
     const hipError_t e = dtype == FDP_BF16 ? launch_wide_bf16(w, wgm, plain, s)
                                            : launch_wide_f16(w, wgm, plain, s);
@@ -616,10 +643,25 @@ int wgrad_clip_impl(const void* a, const void* b, int64_t B, int64_t K, int64_t 
   }
   // fp32: the plan that the workspace query sized, or, in a smaller workspace,
   // the one that fits the least accepted size (the caller forms the bias)
-  const F32Layout fl = f32_layout(B, K, M, N, layout, cus, pl0.groups, false);
+  const F32Layout fl = f32_layout(B, K, M, N, layout, cus, pl0.groups, flags, false);
+  // Paired single pass: aligned rows, every product once.
+  if (!noclip && fl.wp.pair != 0 && fl.total_pair <= workspace_bytes && vec &&
+      lda < (int64_t(1) << 29) && ldb < (int64_t(1) << 29) && stride_ab < (int64_t(1) << 29) &&
+      stride_bb < (int64_t(1) << 29) && pair_records_fit(K, 2 * lda, 2 * stride_ab) &&
+      pair_records_fit(K, 2 * ldb, 2 * stride_bb)) {
+    const WideArgs w = wide_args(fl.wp, true, kWsHead, fl.off_slots, fl.off_bias_part, fl.off_bias_sq);
+    clear_head();
+    e = launch_pair_f32(w, (flags & FDP_WGRAD_PLAIN_LAUNCH) != 0, s);
+    if (e == hipSuccess) {
+      if (bias_done != nullptr) *bias_done = bias != nullptr;
+      return FDP_OK;
+    }
+    (void)hipGetLastError();
+    if (e != hipErrorNotSupported && e != hipErrorCooperativeLaunchTooLarge) return FDP_ERR_HIP;
+  }
   const F32Layout f = fl.total <= workspace_bytes
                           ? fl
-                          : f32_layout(B, K, M, N, layout, cus, pl0.groups, true);
+                          : f32_layout(B, K, M, N, layout, cus, pl0.groups, flags, true);
   args.bias_op = 0;
   args.partials = reinterpret_cast<float*>(ws + f.off_partials);
   args.factors = reinterpret_cast<float*>(ws + f.off_factors);

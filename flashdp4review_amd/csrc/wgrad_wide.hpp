@@ -670,6 +670,115 @@ struct PairGeom {
   static_assert(LOADS_A * NW * 64 * 16 == TILE_A && LOADS_B * NW * 64 * 16 == TILE_B,
                 "each wave issues whole 1 KB loads");
 };
+// The same LDS stage for fp32 operands: rows of 2 x 192 floats, k-tiles of 16
+// (widths count 16-bit units, as the DMA loads do).
+struct PairGeomF32 : PairGeom {
+  static constexpr int BM = 768, BN = 768;
+  static constexpr int BK = 16;
+  static constexpr int KS = BK / 2;  // v_mfma_f32_32x32x2_f32 steps
+  static constexpr int ROW_A = dma::row_chunks(BM) * 16;
+  static constexpr int ROW_B = dma::row_chunks(BN) * 16;
+  static_assert(BK * ROW_A == TILE_A && BK * ROW_B == TILE_B, "the stage of the 16-bit kernel");
+};
+
+// One k-pair's fragments: a lane holds one float of each 32-row block of its
+// wave tile (row lane % 32, k = lane / 32).
+struct PairFragsF32 {
+  float a[3], b[3];
+};
+
+// acc += the wave's 96 x 96 product of its sample (wm / wn: its first LDS
+// columns), as dma::gemm_pipe does it: a 3-stage ring filled by LDS DMA, the
+// next step's fragments read before this step's MFMAs, a freed stage refilled
+// behind its k-tile's last MFMAs.  fhook(kt, ks, frags) as there.
+// An LDS row's chunk c lies at c ^ swz(k), and a step reads rows 2 ks and
+// 2 ks + 1: two bases per block (even and odd steps), set once per k-tile, and
+// constant offsets from them: no address arithmetic beside the MFMAs (every
+// vector instruction delays the next one, see wgrad_f32.hpp).
+template <int S, class J, class FragHook>
+__device__ __forceinline__ void pair_gemm_f32(const J& job, int nk, int wm, int wn,
+                                              const dma::Stages& st, f32x16 (&acc)[3][3],
+                                              const FragHook& fhook) {
+  using G = PairGeomF32;
+  const int lane = threadIdx.x & 63;
+  uint32_t oa[3][2], ob[3][2];
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int k = 2 * h + (lane >> 5);
+      const int ca = wm + 32 * i + (lane & 31), cb = wn + 32 * i + (lane & 31);
+      oa[i][h] = static_cast<uint32_t>(k * G::ROW_A + (((ca >> 2) ^ dma::swz(k)) << 4) + (ca & 3) * 4);
+      ob[i][h] = static_cast<uint32_t>(G::TILE_A + k * G::ROW_B +
+                                       (((cb >> 2) ^ dma::swz(k)) << 4) + (cb & 3) * 4);
+    }
+  const FDP_LDS float *pa[3][2], *pb[3][2];
+  auto enter = [&](const FDP_LDS char* stage) {  // the stage the following loads read
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        pa[i][h] = reinterpret_cast<const FDP_LDS float*>(stage + oa[i][h]);
+        pb[i][h] = reinterpret_cast<const FDP_LDS float*>(stage + ob[i][h]);
+        asm volatile("" : "+v"(pa[i][h]));
+        asm volatile("" : "+v"(pb[i][h]));
+      }
+  };
+  auto load = [&](PairFragsF32& f, int ks) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      f.a[i] = pa[i][ks & 1][(ks >> 1) * G::ROW_A];
+      f.b[i] = pb[i][ks & 1][(ks >> 1) * G::ROW_B];
+    }
+  };
+  dma::wait_vm<0>();
+#pragma unroll
+  for (int s = 0; s < S - 1; ++s)
+    if (s < nk) job.issue(st.get(s), s);
+  if (nk <= 0) return;
+  dma::wait_tiles<G::LOADS>(nk - 1 < S - 2 ? nk - 1 : S - 2);
+  dma::barrier();
+  if (S - 1 < nk) job.issue(st.get(S - 1), S - 1);
+  PairFragsF32 f[2];
+  enter(st.get(0));
+  load(f[0], 0);
+  for (int base = 0; base < nk; base += S) {
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const int kt = base + s;
+      if (kt < nk) {
+#pragma unroll
+        for (int ks = 0; ks < G::KS; ++ks) {
+          const int cur = ks & 1;
+          if (ks + 1 < G::KS) {
+            load(f[cur ^ 1], ks + 1);
+          } else if (kt + 1 < nk) {
+            const int ahead = nk - 2 - kt;
+            dma::wait_tiles<G::LOADS>(ahead < S - 2 ? ahead : S - 2);
+            dma::barrier();
+            enter(st.get((s + 1) % S));
+            load(f[cur ^ 1], 0);
+          }
+#pragma unroll
+          for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(f[cur].a[i], f[cur].b[j], acc[i][j],
+                                                               0, 0, 0);
+#pragma unroll
+          for (int t = 0; t < 9; ++t) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // then a DS read
+          }
+          if (ks + 1 == G::KS && kt + S < nk) job.issue(st.get(s), kt + S);
+          fhook(kt, ks, f[cur]);
+        }
+      }
+    }
+  }
+  dma::barrier();
+}
+
 constexpr int kPairTile = 192;
 constexpr int kPairBlocks = 36;      // 32x32 blocks per 192x192 tile
 constexpr int kPairMinB = 6;         // regions of at most 12 blocks (48 KB in fp32)
@@ -690,7 +799,9 @@ __device__ __forceinline__ int pair_region_first(int q, int ng) {
 template <class DT, int BOP>
 __global__ __launch_bounds__(kWideThreads, 1) void wgrad_pair_kernel(WideArgs p) {
   constexpr bool BIAS = BOP != 0;
-  using G = PairGeom;
+  constexpr bool F32IN = DT::code == FDP_F32;
+  using G = std::conditional_t<F32IN, PairGeomF32, PairGeom>;
+  constexpr int XW = F32IN ? 2 : 1;  // 16-byte words of 8 exchanged values: fp32 or bf16
   constexpr int S = kWideStages;
   __shared__ __attribute__((aligned(16))) char st0[G::STAGE];
   __shared__ __attribute__((aligned(16))) char st1[G::STAGE];
@@ -739,18 +850,25 @@ __global__ __launch_bounds__(kWideThreads, 1) void wgrad_pair_kernel(WideArgs p)
   const int tile_m = static_cast<int>(m0 / kPairTile), tile_n = static_cast<int>(n0 / kPairTile);
   const int blim = bias_limit(BOP == 1 ? p.M : p.N, BOP == 1 ? m0 : n0);
   float bcs[3] = {0.f, 0.f, 0.f}, bsq = 0.f;
-  auto fhook = [&](int kt, int ks, const dma::Frags<G>& f) {
+  // (fp32: of the two waves that share a fragment, each sums every other step)
+  auto count = [&](const auto& x, int c, float& cs) {
+    if constexpr (F32IN) {
+      cs += x;
+      bsq += c < blim ? x * x : 0.f;
+    } else {
+      bias_frag<DT>(x, cs, bsq, c, blim);
+    }
+  };
+  auto fhook = [&](int kt, int ks, const auto& f) {
     if constexpr (BOP == 1) {
-      if (kt % p.tiles_n == tile_n && (wl & 1) == ks) {
+      if (kt % p.tiles_n == tile_n && (wl & 1) == (ks & 1)) {
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
-          bias_frag<DT>(f.a[i], bcs[i], bsq, wm + 32 * i + (lane & 31), blim);
+        for (int i = 0; i < 3; ++i) count(f.a[i], wm + 32 * i + (lane & 31), bcs[i]);
       }
     } else if constexpr (BOP == 2) {
-      if (kt % p.tiles_m == tile_m && (wl >> 1) == ks) {
+      if (kt % p.tiles_m == tile_m && (wl >> 1) == (ks & 1)) {
 #pragma unroll
-        for (int j = 0; j < 3; ++j)
-          bias_frag<DT>(f.b[j], bcs[j], bsq, wn + 32 * j + (lane & 31), blim);
+        for (int j = 0; j < 3; ++j) count(f.b[j], wn + 32 * j + (lane & 31), bcs[j]);
       }
     }
   };
@@ -763,7 +881,13 @@ __global__ __launch_bounds__(kWideThreads, 1) void wgrad_pair_kernel(WideArgs p)
     for (int j = 0; j < 3; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-  {
+  if constexpr (F32IN) {
+    dma::PairJob<G> job;  // (p.a and p.b point at floats: 16-bit units are half of one)
+    job.init(p.a + 2 * s0 * p.sab, 2 * p.lda, 2 * p.sab, p.b + 2 * s0 * p.sbb, 2 * p.ldb,
+             2 * p.sbb, p.K, 2 * m0, 2 * n0);
+    pair_gemm_f32<S>(job, static_cast<int>(p.K / G::BK), half * kPairTile + wm,
+                     half * kPairTile + wn, stages, acc, fhook);
+  } else {
     dma::FragOffsets<G> fo;
     fo.init(half * kPairTile + wm, half * kPairTile + wn);
     dma::PairJob<G> job;
@@ -932,7 +1056,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void wgrad_pair_kernel(WideArgs p)
   const float cmine = fac[half];
   f32x4* const stg[2] = {reinterpret_cast<f32x4*>(st0), reinterpret_cast<f32x4*>(st2)};
   f32x4* own = reinterpret_cast<f32x4*>(st1);
-  const int slot_bytes = p.slot_blocks * kWideBlockBytes;
+  const int slot_bytes = p.slot_blocks * kWideBlockBytes * XW;
   {
     const CoherentSpan slot(reinterpret_cast<const float*>(p.slots + int64_t(L) * slot_bytes),
                             static_cast<uint32_t>(slot_bytes));
@@ -969,12 +1093,17 @@ __global__ __launch_bounds__(kWideThreads, 1) void wgrad_pair_kernel(WideArgs p)
             o[0] = f32x4{v[8 * h], v[8 * h + 1], v[8 * h + 2], v[8 * h + 3]};
             o[1] = f32x4{v[8 * h + 4], v[8 * h + 5], v[8 * h + 6], v[8 * h + 7]};
           } else {
-            u32x4 w;
+            const uint32_t at = static_cast<uint32_t>(
+                ((slot_block(bid, rb0, rb1) * 2 + h) * XW) * 1024 + lane * 16);
+            if constexpr (F32IN) {
+              slot.store4(at, f32x4{v[8 * h], v[8 * h + 1], v[8 * h + 2], v[8 * h + 3]});
+              slot.store4(at + 1024, f32x4{v[8 * h + 4], v[8 * h + 5], v[8 * h + 6], v[8 * h + 7]});
+            } else {
+              u32x4 w;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) w[e] = BF16::pack2(v[8 * h + 2 * e], v[8 * h + 2 * e + 1]);
-            slot.store4(
-                static_cast<uint32_t>((slot_block(bid, rb0, rb1) * 2 + h) * 1024 + lane * 16),
-                __builtin_bit_cast(f32x4, w));
+              for (int e = 0; e < 4; ++e) w[e] = BF16::pack2(v[8 * h + 2 * e], v[8 * h + 2 * e + 1]);
+              slot.store4(at, __builtin_bit_cast(f32x4, w));
+            }
           }
         }
       }
@@ -1024,12 +1153,20 @@ __global__ __launch_bounds__(kWideThreads, 1) void wgrad_pair_kernel(WideArgs p)
   const int64_t slot_stride = int64_t(p.tiles) * slot_bytes;  // between pairs of one tile
   const char* const slots_tile = p.slots + int64_t(tile) * slot_bytes;
   float* const rows = reinterpret_cast<float*>(st0);
-  auto slot_load = [&](int qq, int it) -> u32x4 {
+  struct Words {
+    u32x4 w[XW];
+  };
+  auto slot_load = [&](int qq, int it) -> Words {
     const int bid = rb0 + (it >> 7), h = (it >> 6) & 1, l = it & 63;
     const CoherentSpan sl(reinterpret_cast<const float*>(slots_tile + qq * slot_stride),
                           static_cast<uint32_t>(slot_bytes));
     const int sb = slot_block(bid, pair_region_first(qq, ng), pair_region_first(qq + 1, ng));
-    return __builtin_bit_cast(u32x4, sl.load4(static_cast<uint32_t>((sb * 2 + h) * 1024 + l * 16)));
+    Words r;
+#pragma unroll
+    for (int x = 0; x < XW; ++x)
+      r.w[x] = __builtin_bit_cast(
+          u32x4, sl.load4(static_cast<uint32_t>(((sb * 2 + h) * XW + x) * 1024 + l * 16)));
+    return r;
   };
   auto add_own = [&](float (&v)[8], int it) {
     const int lb = it >> 7, h = (it >> 6) & 1, l = it & 63;
@@ -1041,7 +1178,16 @@ __global__ __launch_bounds__(kWideThreads, 1) void wgrad_pair_kernel(WideArgs p)
       v[4 + e] += hi[e];
     }
   };
-  auto add_bf16 = [&](float (&v)[8], const u32x4& w) {
+  auto add_words = [&](float (&v)[8], const Words& x) {
+    if constexpr (F32IN) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] += __uint_as_float(x.w[0][e]);
+        v[4 + e] += __uint_as_float(x.w[XW - 1][e]);
+      }
+      return;
+    }
+    const u32x4& w = x.w[0];
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
       v[2 * e] += __uint_as_float(w[e] << 16);
@@ -1061,10 +1207,10 @@ __global__ __launch_bounds__(kWideThreads, 1) void wgrad_pair_kernel(WideArgs p)
   };
   constexpr int R = (kPairRegionMax * 128 + kWideThreads - 1) / kWideThreads;
   static_assert(R == 3, "three rounds of items per thread at most");
-  if (ng <= kPairFast) {
+  if (!F32IN && ng <= kPairFast) {  // (fp32 words of every round would not fit the registers)
     // every chunk of every item of this thread in flight at once (at most
     // R x (kPairFast - 1) loads), then the sums
-    u32x4 w[R][kPairFast];
+    Words w[R][kPairFast];
 #pragma unroll
     for (int k = 0; k < R; ++k) {
       const int it = threadIdx.x + k * kWideThreads;
@@ -1084,7 +1230,9 @@ __global__ __launch_bounds__(kWideThreads, 1) void wgrad_pair_kernel(WideArgs p)
       for (int qq = 0; qq < kPairFast; ++qq) {
         if (qq >= ng) break;
         if (qq == q) add_own(v, it);
-        else add_bf16(v, k == 0 ? w[0][qq] : k == 1 ? w[1][qq] : w[2][qq]);
+        else if (k == 0) add_words(v, w[0][qq]);
+        else if (k == 1) add_words(v, w[1][qq]);
+        else add_words(v, w[2][qq]);
       }
       put_rows(it, v);
     }
@@ -1095,7 +1243,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void wgrad_pair_kernel(WideArgs p)
       // chunks in pair order, kPairFast loads in flight at a time
 #pragma unroll 1
       for (int qb = 0; qb < ng; qb += kPairFast) {
-        u32x4 w[kPairFast];
+        Words w[kPairFast];
 #pragma unroll
         for (int u = 0; u < kPairFast; ++u)
           if (qb + u < ng && qb + u != q) w[u] = slot_load(qb + u, it);
@@ -1103,7 +1251,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void wgrad_pair_kernel(WideArgs p)
         for (int u = 0; u < kPairFast; ++u) {
           if (qb + u >= ng) break;
           if (qb + u == q) add_own(v, it);
-          else add_bf16(v, w[u]);
+          else add_words(v, w[u]);
         }
       }
       put_rows(it, v);
@@ -1306,9 +1454,15 @@ struct WidePlan {
 inline bool pair_records_fit(int64_t K, int64_t ld, int64_t ds) {
   return fits_record(K, ld, ds);
 }
+// f32: fp32 operands (strides in floats), which only the paired kernel takes.
 inline WidePlan wide_plan(int64_t B, int64_t K, int64_t M, int64_t N, int64_t lda, int64_t ldb,
-                          int cus, double min_fill) {
+                          int cus, double min_fill, bool f32 = false) {
   WidePlan w{};
+  if (f32 && (lda >= (int64_t(1) << 29) || ldb >= (int64_t(1) << 29))) return w;
+  if (f32) {  // in 16-bit units, as the records count
+    lda *= 2;
+    ldb *= 2;
+  }
   if (!fits_record(K, lda) || !fits_record(K, ldb)) return w;
   const double fill = double(M) * double(N) * double(B) / (double(cus) * 73728.0);
   if (fill < min_fill) return w;
@@ -1325,7 +1479,7 @@ inline WidePlan wide_plan(int64_t B, int64_t K, int64_t M, int64_t N, int64_t ld
   }
   w.tiles = static_cast<int>(best_tiles);
   const int64_t units = best_tiles * B;
-  if (units > cus || B < 2 || B > kWideBlocks) {
+  if (f32 || units > cus || B < 2 || B > kWideBlocks) {
     w.wgm = 0;
   } else {
     w.nwg = static_cast<int>(units);
@@ -1338,7 +1492,8 @@ inline WidePlan wide_plan(int64_t B, int64_t K, int64_t M, int64_t N, int64_t ld
   }
   const int64_t ptm = (M + kPairTile - 1) / kPairTile, ptn = (N + kPairTile - 1) / kPairTile;
   const int64_t punits = ptm * ptn * (B / 2);
-  if (B % 2 == 0 && B >= kPairMinB && B <= 2 * kPairBlocks && K % PairGeom::BK == 0 &&
+  if (B % 2 == 0 && B >= kPairMinB && B <= 2 * kPairBlocks &&
+      K % (f32 ? PairGeomF32::BK : PairGeom::BK) == 0 &&
       ptm * ptn + 1 <= kGroupMax && punits <= cus && pair_records_fit(K, lda, K * lda) &&
       pair_records_fit(K, ldb, K * ldb)) {
     w.pair = 1;
@@ -1349,7 +1504,7 @@ inline WidePlan wide_plan(int64_t B, int64_t K, int64_t M, int64_t N, int64_t ld
     const int ng = static_cast<int>(B / 2);
     w.pair_slot_blocks = kPairBlocks - kPairBlocks / ng;
     const size_t pb = sizeof(uint64_t) * size_t(B) * w.pair_tiles;
-    const size_t sb = size_t(punits) * size_t(w.pair_slot_blocks) * kWideBlockBytes;
+    const size_t sb = size_t(punits) * size_t(w.pair_slot_blocks) * kWideBlockBytes * (f32 ? 2 : 1);
     // bias: [tiles_own * 192][B][P] words with tiles_own * P = the tile count
     const size_t bp = sizeof(uint64_t) * size_t(kPairTile) * size_t(B) * w.pair_tiles;
     const size_t bq = sizeof(uint64_t) * size_t(B) * w.pair_tiles;
@@ -1384,6 +1539,8 @@ hipError_t launch_wide_t(const WideArgs& a, int wgm, bool plain, hipStream_t s) 
                : hipLaunchCooperativeKernel(fn, dim3(a.nwg), dim3(kWideThreads), params, 0, s);
 }
 
+// The paired kernel for fp32 operands (wgrad_pair_f32.hip).
+hipError_t launch_pair_f32(const WideArgs& a, bool plain, hipStream_t s);
 hipError_t launch_wide_bf16(const WideArgs& a, int wgm, bool plain, hipStream_t s);
 hipError_t launch_wide_f16(const WideArgs& a, int wgm, bool plain, hipStream_t s);
 

@@ -123,3 +123,73 @@ def test_f32_noise_strides_and_least_workspace(shape, out_dtype):
         assert st == 0
         outs.append(out)
         assert_close(out, ref / B, torch.float32, f"{nbytes} bytes")
+
+
+PAIR_SHAPES = [  # B, K, M, N: even batches, whole 16-deep k-tiles, 16-byte aligned rows
+    (6, 16, 64, 64),        # one k-tile, part of one tile
+    (6, 32, 192, 192),      # one whole tile
+    (8, 48, 392, 520),      # ring wraps at three k-tiles, ragged tiles
+    (8, 128, 196, 768),
+    (24, 64, 200, 380),     # more pairs than load at once
+    (72, 16, 64, 192),      # the largest batch: one block per region
+    (8, 64, 1536, 1536),    # fills the device: the default route
+]
+
+
+@pytest.mark.parametrize("bias", [None, "a", "b"])
+@pytest.mark.parametrize("shape", PAIR_SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_f32_paired(shape, bias):
+    """The paired single pass on fp32 operands ("wide": wherever its plan
+    applies): sum, norms and factors and the bias of either operand at the fp32
+    bar, with the drawn noise, repeated bitwise, beside two-pass calls on the
+    same workspace."""
+    B, K, M, N = shape
+    a, b = make(B, K, M, N, "tn", seed=7)
+    _, norms_ref, _ = O.wgrad_clip(a, b, 1.0, 1.0, "tn")
+    C = float(np.median(norms_ref))
+    ref, norms_ref, fac_ref = O.wgrad_clip(a, b, C, 1.0, "tn")
+    kw = dict(out_scale=1.0 / B, noise_scale=0.01, noise_key=(5, 9), single_pass="wide",
+              return_stats=True, check=True)
+    n = M if bias == "a" else N
+    db = torch.empty(n, device=DEV)
+    if bias is not None:
+        kw.update(bias_out=db, bias_scale=0.25, bias_operand=bias, bias_noise_scale=0.02,
+                  bias_noise_key=(6, 1))
+    r = core.wgrad_clip(a, b, C, 1.0, **kw)
+    expect = ref / B + 0.01 * philox.normals(M * N, 5, 9).reshape(M, N)
+    assert_close(r[0], expect, torch.float32, "sum")
+    assert_elementwise(r[1], norms_ref, torch.float32, "norms")
+    assert_elementwise(r[2], fac_ref, torch.float32, "factors")
+    first_db = db.clone()
+    two = core.wgrad_clip(a, b, C, 1.0, out_scale=1.0 / B, two_pass=True)
+    assert_close(two, ref / B, torch.float32, "two passes")
+    again = core.wgrad_clip(a, b, C, 1.0, **kw)
+    assert torch.equal(again[0], r[0])
+    if bias is not None:
+        u = (a if bias == "a" else b).double().cpu().numpy()
+        nr = np.sqrt((u ** 2).sum((1, 2)))
+        assert_elementwise(r[3], nr, torch.float32, "bias norms")
+        fac = np.minimum(1.0, C / (nr + 1e-10))
+        assert_close(first_db, 0.25 * (fac[:, None] * u.sum(1)).sum(0) + 0.02 * philox.normals(n, 6, 1),
+                     torch.float32, "bias")
+        assert torch.equal(first_db, db)
+
+
+def test_f32_paired_strides_and_expiry(monkeypatch):
+    """Samples two apart and rows inside wider ones, with infinities around; and a
+    wait that gives up at once: NaN, an error, and a correct next call."""
+    B, K, M, N = 6, 32, 64, 72
+    wa = torch.full((2 * B, K, M + 8), float("inf"), device=DEV)
+    wb = torch.full((2 * B, K, N + 4), float("inf"), device=DEV)
+    a0, b0 = make(B, K, M, N, "tn", seed=8)
+    a, b = wa[::2, :, 4:M + 4], wb[::2, :, :N]
+    a.copy_(a0)
+    b.copy_(b0)
+    ref, _, _ = O.wgrad_clip(a0, b0, 1.0, 1.0, "tn")
+    assert_close(core.wgrad_clip(a, b, 1.0, 1.0, single_pass="wide"), ref, torch.float32)
+    monkeypatch.setenv("FDP_WGRAD_SPIN_LIMIT", "0")
+    with pytest.raises(_lib.FlashDPError):
+        core.wgrad_clip(a0, b0, 1.0, 1.0, single_pass="wide", check=True)
+    monkeypatch.delenv("FDP_WGRAD_SPIN_LIMIT")
+    out = core.wgrad_clip(a0, b0, 1.0, 1.0, single_pass="wide", check=True)
+    assert_close(out, ref, torch.float32, "after the expiry")
