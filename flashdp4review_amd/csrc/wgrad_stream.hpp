@@ -631,11 +631,22 @@ inline StreamPlan stream_plan(int64_t B, int64_t K, int64_t M, int64_t N, int cu
   s.gram_per_sample = s.gram_nt * (s.gram_nt + 1) / 2;
   const double direct = double(K) * M * N;
   const double gram = double(s.gram_per_sample) * kGramT * kGramT * double(M + N);
-  s.gram = M % 64 == 0 && N % 64 == 0 && K > 0 && gram < direct;
+  // Aligned TN operands take the Gram form where it is estimated faster than the
+  // products, not only smaller: a short batch has few Gram tiles, each a serial
+  // walk over every feature.  Us, from kernel times with two workgroups per CU: a
+  // 64-deep Gram k-tile 0.9, a 32-deep one of the products 0.9 and 3 per round of
+  // tiles (8 x 1024, 2048 -> 8192: 144 against 254; 1 x 22, 1472 -> 7232, one Gram
+  // tile: 122 against 4).
+  const double slots = 2. * cus;
+  const double gram_us =
+      std::ceil(double(B) * s.gram_per_sample / slots) * double(M + N) / 64 * 0.9;
+  const double prod_us = std::ceil(double(s.norm.tiles()) * B / slots) *
+                         (static_cast<double>((K + 31) / 32) * 0.9 + 3.);
+  s.gram = M % 64 == 0 && N % 64 == 0 && K > 0 && gram_us < prod_us;
   // the split Gram norm (wgrad_staged.hpp): the longer operand's Gram tiles are
   // contracted in parts until there are two workgroups per CU, of at least 8
   // k-tiles each, with at most 64 MB of partial tiles
-  const double items = double(B) * s.gram_per_sample, slots = 2. * cus;
+  const double items = double(B) * s.gram_per_sample;
   if ((M % 8 != 0 || N % 8 != 0) && K > 0 && gram < 0.8 * direct &&
       items * kGramPartBytes <= 64e6) {
     const double longer = double((M > N ? M : N) + 63) / 64, shorter = double((M > N ? N : M) + 63) / 64;

@@ -128,7 +128,8 @@ int fdp_version(void);
  *            contiguous.  The single-pass and streamed kernels address one
  *            sample's operand through a 32-bit buffer record: a sample whose
  *            K (rounded up to 128) times its row stride reaches 2^30 elements
- *            takes the generic two-pass schedule (64-bit addressing) instead.
+ *            takes the two-pass schedule that loads through registers with
+ *            64-bit addressing instead.
  * out      : [M, N] row-major with row stride ldo, dtype `out_dtype`.
  * noise    : NULL or [M, N] contiguous, dtype `out_dtype`.
  * noise_key: NULL, or the in-kernel draw used when `noise` is NULL.

@@ -89,3 +89,40 @@ def test_last_rows_of_an_allocation():
         views.append(v)
     out = core.wgrad_clip(*views, 1.0, 1.0, out_dtype=torch.float32, two_pass=True)
     assert_close(out, ref, torch.float32)
+
+
+ROUTES = [  # B, K, M, N, whether the default is the two-pass schedule
+    # few Gram tiles: norms from the products; many: the Gram form
+    (1, 22, 1472, 7232, True),
+    (8, 150, 2240, 5120, True),
+]
+
+
+@pytest.mark.parametrize("route", ROUTES, ids=lambda s: "x".join(map(str, s[:4])))
+def test_default_route(route):
+    """The rule between Gram and product norms: the oracle's result on either side."""
+    B, K, M, N, two = route
+    g = torch.Generator(DEV).manual_seed(B * K)
+    a = torch.randn(B, K, M, generator=g, device=DEV).to(torch.bfloat16)
+    b = torch.randn(B, K, N, generator=g, device=DEV).to(torch.bfloat16)
+    # per-sample scales, powers of two: exact in bf16, and clipped and unclipped samples
+    b *= torch.tensor([2.0 ** (i % 3) for i in range(B)], device=DEV).to(b.dtype).view(B, 1, 1)
+    C = 2.0 * (K * M * N) ** 0.5
+    ref = torch.zeros(M, N, dtype=torch.float64, device=DEV)
+    norms_ref, fac_ref = [], []
+    for i in range(B):
+        G = a[i].double().t() @ b[i].double()
+        norms_ref.append(G.norm())
+        fac_ref.append((C / norms_ref[-1]).clamp(max=1.0))
+        ref += fac_ref[-1] * G
+    kw = dict(out_dtype=torch.float32, return_stats=True)
+    out, norms, fac = core.wgrad_clip(a, b, C, 1.0, **kw)
+    forced, _, _ = core.wgrad_clip(a, b, C, 1.0, two_pass=True, **kw)
+    if two:
+        assert torch.equal(out, forced)
+        assert_close(out, ref.cpu().numpy(), torch.float32, "sum")
+    else:  # the single pass parks its products in 16 bits
+        assert_close(out, ref.cpu().numpy(), torch.bfloat16, "sum")
+        assert_close(forced, ref.cpu().numpy(), torch.float32, "two-pass sum")
+    assert_elementwise(norms, torch.stack(norms_ref).cpu().numpy(), torch.float32, "norms")
+    assert_elementwise(fac, torch.stack(fac_ref).cpu().numpy(), torch.float32, "factors")
