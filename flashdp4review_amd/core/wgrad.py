@@ -9,6 +9,7 @@ point, ``wgrad_clip``, which never materialises a per-sample gradient.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import threading
 
@@ -236,6 +237,35 @@ def set_wgrad_launch(mode: str) -> str:
     return prev
 
 
+@functools.lru_cache(maxsize=None)
+def _num_cus(index):
+    return torch.cuda.get_device_properties(index).multi_processor_count
+
+
+def _two_pass_pays(B, K, M, N, cus):
+    """Whether the streamed two-pass schedule is the faster one for 16-bit operands
+    that the grouped single pass would take (layout "tn", aligned rows; others take
+    two passes either way).
+
+    A single-pass launch pays its grid barrier, its parked 16-bit products and, with
+    several launches, a read and a write of the fp32 gradient per four samples; two
+    passes pay a second contraction, little where K is short.  Over 250 drawn shapes,
+    bf16, single pass against two passes, us (B x K, M x N): one launch whose
+    workgroups hold several samples breaks even near K = 64 (6 x 23, 1216 x 1088: 36
+    against 22; 15 x 25, 1344 x 768: 56 against 39; 4 x 80, 1408 x 3264: 35 against 37;
+    3 x 200, 1216 x 3392: 36 against 45), several launches near K = 400 (30 x 59, 3136 x
+    1536: 258 against 81; 37 x 256, 1616 x 1672: 203 against 153; 6 x 320, 4504 x 1760:
+    114 against 99; 44 x 512, 1952 x 872: 165 against 204), or 600 where one sample has
+    more tiles than CUs (33 x 512, 1728 x 3776: 531 against 350; 32 x 1000, 1816 x 3896:
+    893 against 938)."""
+    tiles, slots = -(-M // 128) * -(-N // 128), 2 * cus
+    if tiles > slots or 0.7 <= B * M * N / (cus * 73728) <= 1.0:
+        return False  # two passes by default, or the wide schedule's range
+    if 4 * (slots // tiles) < B:
+        return K <= (600 if tiles > cus else 400)
+    return tiles * B > slots and K <= 64
+
+
 class _Prepared:
     """A checked call signature of wgrad_clip (contiguous operands, no injected
     noise, no stats): the per-call work left is the output allocation, the
@@ -332,7 +362,7 @@ def wgrad_clip(a: torch.Tensor, b: torch.Tensor, C: float = 1.0, clamp_value: fl
     ``two_pass`` forces the norm-pass + clipped-sum-pass schedule instead of the
     single-pass kernels; ``single_pass`` picks between those: "auto" (the wide
     schedule when the layer's products fill at least 70% of the CUs, else the
-    grouped 128x128 kernel), "wide" (the wide schedule whenever the products
+    grouped 128x128 kernel, or two passes where K is short for it), "wide" (the wide schedule whenever the products
     fit the CUs), "unpaired" (as "wide", one sample per CU only) or "narrow"
     (grouped only).  The wide schedule holds two samples' 192x192 tiles per CU
     where the batch is even (6..72) and the contraction a multiple of 32 (a
@@ -436,6 +466,9 @@ def wgrad_clip(a: torch.Tensor, b: torch.Tensor, C: float = 1.0, clamp_value: fl
         raise ValueError(f"launch must be one of {_LAUNCH_MODES}, got {mode!r}")
     if single_pass not in _SINGLE_PASS:
         raise ValueError(f"single_pass must be one of {tuple(_SINGLE_PASS)}, got {single_pass!r}")
+    if (single_pass == "auto" and not two_pass and not noclip and layout == "tn"
+            and a.dtype != torch.float32 and _two_pass_pays(Bn, K, M, N, _num_cus(dev.index))):
+        two_pass = True
     flags = ((_lib.WGRAD_NOCLIP if noclip else 0) | (_lib.WGRAD_TWO_PASS if two_pass else 0)
              | (_lib.WGRAD_PLAIN_LAUNCH if mode == "plain" else 0) | _lib.WGRAD_CLEAN_WORKSPACE
              | _SINGLE_PASS[single_pass]

@@ -92,15 +92,27 @@ def test_last_rows_of_an_allocation():
 
 
 ROUTES = [  # B, K, M, N, whether the default is the two-pass schedule
+    # several samples per workgroup in one launch (100 tiles): K of 64 and 65
+    (6, 64, 1280, 1280, True),
+    (6, 65, 1280, 1280, False),
+    (5, 64, 1280, 1280, False),    # 500 workgroups, one sample each
+    (7, 1, 1216, 1224, True),
+    # several launches (21 samples each of 24 tiles; 4 of 289): K at the two limits
+    (85, 400, 512, 768, True),
+    (85, 401, 512, 768, False),
+    (5, 600, 2120, 2120, True),
+    (5, 601, 2120, 2120, False),
     # few Gram tiles: norms from the products; many: the Gram form
     (1, 22, 1472, 7232, True),
     (8, 150, 2240, 5120, True),
+    (40, 70, 2048, 1024, True),
 ]
 
 
 @pytest.mark.parametrize("route", ROUTES, ids=lambda s: "x".join(map(str, s[:4])))
 def test_default_route(route):
-    """The rule between Gram and product norms: the oracle's result on either side."""
+    """The rule between the grouped single pass and the two passes, and the one
+    between Gram and product norms: the oracle's result on either side."""
     B, K, M, N, two = route
     g = torch.Generator(DEV).manual_seed(B * K)
     a = torch.randn(B, K, M, generator=g, device=DEV).to(torch.bfloat16)
