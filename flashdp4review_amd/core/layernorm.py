@@ -12,6 +12,7 @@ layernorm_dwdb_fused reduces those rows to the parameter dtype.
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 
@@ -32,6 +33,12 @@ def check_fused_row(x: torch.Tensor) -> None:
     64 KB (flashdp/core/layernorm_clip.py:217-221)."""
     if x.shape[-1] * x.element_size() > FUSED_MAX_ROW_BYTES:
         raise RuntimeError("This layer norm doesn't support feature dim >= 64KB.")
+
+
+@functools.lru_cache(maxsize=1024)
+def _bwd_workspace_bytes(B: int, T: int, H: int, dt: int, index: int) -> int:
+    """Workspace of the backward; it depends on the sizes and the device only."""
+    return _lib.size_query(_lib.lib().fdp_layernorm_bwd_clip_workspace_size, B, T, H, dt)
 
 
 def _rows(x: torch.Tensor, H: int) -> int:
@@ -55,10 +62,14 @@ def layernorm_fwd(x: torch.Tensor, weight: torch.Tensor | None, bias: torch.Tens
     y = torch.empty_like(x)
     mean = torch.empty(rows, dtype=torch.float32, device=dev)
     rstd = torch.empty(rows, dtype=torch.float32, device=dev)
-    L = _lib.lib()
-    st = L.fdp_layernorm_fwd(_lib.ptr(x), _lib.ptr(weight), _lib.ptr(bias), rows, H,
-                             ctypes.c_float(eps), dt, wdt, y.data_ptr(), mean.data_ptr(),
-                             rstd.data_ptr(), _lib.stream_handle(dev))
+    fast = _lib.fast_call()
+    if fast is not None:
+        st = fast.ln_fwd(x.data_ptr(), _lib.ptr(weight), _lib.ptr(bias), rows, H, eps, dt, wdt,
+                         y.data_ptr(), mean.data_ptr(), rstd.data_ptr(), _lib.stream_handle(dev))
+    else:
+        st = _lib.lib().fdp_layernorm_fwd(
+            _lib.ptr(x), _lib.ptr(weight), _lib.ptr(bias), rows, H, ctypes.c_float(eps), dt, wdt,
+            y.data_ptr(), mean.data_ptr(), rstd.data_ptr(), _lib.stream_handle(dev))
     _lib.check(st, "fdp_layernorm_fwd")
     return y, mean, rstd
 
@@ -106,16 +117,24 @@ def layernorm_bwd_clip(grad_output: torch.Tensor, x: torch.Tensor, weight: torch
     if return_stats:
         norms = torch.empty(2 * B, dtype=torch.float32, device=dev)
         factors = torch.empty(2 * B, dtype=torch.float32, device=dev)
-    L = _lib.lib()
-    ws = _lib.workspace(
-        _lib.size_query(L.fdp_layernorm_bwd_clip_workspace_size, B, T, H, dt), dev)
-    st = L.fdp_layernorm_bwd_clip(
-        dy.data_ptr(), x.data_ptr(), _lib.ptr(weight), mean.data_ptr(), rstd.data_ptr(), B, T, H,
-        dt, wdt, ctypes.c_float(C_), ctypes.c_float(clamp_), _lib.ptr(cad),
-        ctypes.c_float(out_scale), _lib.ptr(noise_w), _lib.ptr(noise_b),
-        ctypes.c_float(noise_scale), _lib.noise_key(noise_key), dx.data_ptr(), _lib.ptr(dw),
-        _lib.ptr(db), _lib.ptr(norms),
-        _lib.ptr(factors), ws.data_ptr(), ws.numel(), _lib.stream_handle(dev))
+    ws = _lib.workspace(_bwd_workspace_bytes(B, T, H, dt, dev.index), dev)
+    fast = _lib.fast_call()
+    if fast is not None:
+        if noise_key is not None:
+            noise_key = (int(noise_key[0]), int(noise_key[1]), *noise_key[2:3])
+        st = fast.ln_bwd(
+            dy.data_ptr(), x.data_ptr(), _lib.ptr(weight), mean.data_ptr(), rstd.data_ptr(), B, T,
+            H, dt, wdt, C_, clamp_, _lib.ptr(cad), out_scale, _lib.ptr(noise_w), _lib.ptr(noise_b),
+            noise_scale, noise_key, dx.data_ptr(), _lib.ptr(dw), _lib.ptr(db), _lib.ptr(norms),
+            _lib.ptr(factors), ws.data_ptr(), ws.numel(), _lib.stream_handle(dev))
+    else:
+        st = _lib.lib().fdp_layernorm_bwd_clip(
+            dy.data_ptr(), x.data_ptr(), _lib.ptr(weight), mean.data_ptr(), rstd.data_ptr(), B, T,
+            H, dt, wdt, ctypes.c_float(C_), ctypes.c_float(clamp_), _lib.ptr(cad),
+            ctypes.c_float(out_scale), _lib.ptr(noise_w), _lib.ptr(noise_b),
+            ctypes.c_float(noise_scale), _lib.noise_key(noise_key), dx.data_ptr(), _lib.ptr(dw),
+            _lib.ptr(db), _lib.ptr(norms), _lib.ptr(factors), ws.data_ptr(), ws.numel(),
+            _lib.stream_handle(dev))
     _lib.check(st, "fdp_layernorm_bwd_clip")
     if return_stats:
         return dx, dw, db, norms, factors
