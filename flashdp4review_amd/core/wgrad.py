@@ -259,8 +259,8 @@ def _two_pass_pays(B, K, M, N, cus):
     more tiles than CUs (33 x 512, 1728 x 3776: 531 against 350; 32 x 1000, 1816 x 3896:
     893 against 938)."""
     tiles, slots = -(-M // 128) * -(-N // 128), 2 * cus
-    if tiles > slots or 0.7 <= B * M * N / (cus * 73728) <= 1.0:
-        return False  # two passes by default, or the wide schedule's range
+    if not 0 < tiles <= slots or 0.7 <= B * M * N / (cus * 73728) <= 1.0:
+        return False  # refused (empty), two passes by default, or the wide schedule's range
     if 4 * (slots // tiles) < B:
         return K <= (600 if tiles > cus else 400)
     return tiles * B > slots and K <= 64

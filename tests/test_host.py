@@ -261,3 +261,12 @@ def test_wrap_leaves_subclasses_and_wrapped_layers_alone(capsys):
     assert isinstance(n.a, DPLayerNorm) and not n.a.use_fused and n.a.bias is None
     assert isinstance(n.b, DPLayerNorm) and not n.b.use_fused and n.b.weight.shape == (4, 8)
     assert isinstance(n.c, DPLayerNorm) and n.c.use_fused and n.c.weight is None
+
+
+def test_two_pass_rule_leaves_empty_layers_to_the_library():
+    """The schedule rule divides by a sample's tiles: a layer without outputs has
+    none, and the library refuses it."""
+    from flashdp4review_amd.core.wgrad import _two_pass_pays
+    assert not _two_pass_pays(4, 16, 0, 64, 256)
+    assert not _two_pass_pays(4, 16, 64, 0, 256)
+    assert _two_pass_pays(30, 59, 3136, 1536, 256)
