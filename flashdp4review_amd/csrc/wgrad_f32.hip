@@ -52,7 +52,7 @@ hipError_t launch_f32(Args a, const F32Plan& f, int layout, bool noclip, hipStre
   const int64_t K = a.K > 0 ? a.K : 1;
   const int64_t nsamp = f.rows_per_split / K + 2;
   a.groups = f.splits;
-  if (noclip) {
+  if (noclip && a.K > 0) {  // (without rows the sum pass meets no sample)
     a.fac_parts = -1;
   } else if (a.K > 0 &&
              (f.per_sample <= kF32FacThread || nsamp * f.per_sample <= 16384)) {

@@ -193,3 +193,17 @@ def test_f32_paired_strides_and_expiry(monkeypatch):
     monkeypatch.delenv("FDP_WGRAD_SPIN_LIMIT")
     out = core.wgrad_clip(a0, b0, 1.0, 1.0, single_pass="wide", check=True)
     assert_close(out, ref, torch.float32, "after the expiry")
+
+
+@pytest.mark.parametrize("noclip", [False, True])
+@pytest.mark.parametrize("layout", ["tn", "nn"])
+def test_f32_samples_without_rows(layout, noclip):
+    """K = 0: zero products, and every sample's statistics are still written."""
+    B, M, N = 5, 70, 129
+    a = torch.empty((B, 0, M) if layout == "tn" else (B, M, 0), device=DEV)
+    b = torch.empty(B, 0, N, device=DEV)
+    out, norms, fac = core.wgrad_clip(a, b, 1.0, 0.75, layout=layout, noclip=noclip,
+                                      return_stats=True)
+    assert torch.count_nonzero(out) == 0
+    assert norms is None if noclip else torch.count_nonzero(norms) == 0
+    assert torch.equal(fac.cpu(), torch.full((B,), 0.75))
