@@ -420,7 +420,7 @@ namespace {
 // fdp_wgrad_clip; with `bias`, the 16-bit TN kernels (wide, grouped and
 // streamed) also form the bias of operand a (bias_op 1) or b (bias_op 2) from
 // the fragments they hold, with its partials in bias_part / bias_sq
-// (*bias_done = true); the generic two-pass schedule leaves it to the caller.
+// (*bias_done = true), as does the fp32 paired one; the others leave it to the caller.
 int wgrad_clip_impl(const void* a, const void* b, int64_t B, int64_t K, int64_t M, int64_t N,
                     int64_t stride_ab, int64_t lda, int64_t stride_bb, int64_t ldb, int layout,
                     int dtype, float C, float clamp, const float* clip_args_dev, float out_scale,
@@ -689,7 +689,7 @@ extern "C" int fdp_wgrad_clip(const void* a, const void* b, int64_t B, int64_t K
 namespace {
 
 // Workspace of fdp_wgrad_bias_clip (every part 256-aligned): the weight
-// gradient's workspace, the column-sum kernel's (the bias when the generic
+// gradient's workspace, the column-sum kernel's (the bias when a register-fed
 // schedule runs), then the bias partials of the grouped and streamed kernels
 // (bias_part [B, P, len], bias_sq [B, tiles], sized for both tile grids).
 struct BiasLayout {
@@ -750,7 +750,7 @@ extern "C" int fdp_wgrad_bias_clip(const void* a, const void* b, int64_t B, int6
   if (bias == nullptr || bias->out == nullptr) return FDP_ERR_ARG;
   if (!valid_dtype(bias->out_dtype)) return FDP_ERR_DTYPE;
   // the bias operand is [B, K, len] over K, contiguous (the column-sum kernel
-  // reads it that way when the generic schedule runs); the clip is not
+  // reads it that way when a register-fed schedule runs); the clip is not
   // optional
   if (layout != FDP_LAYOUT_TN || (flags & FDP_WGRAD_NOCLIP) != 0) return FDP_ERR_ARG;
   if (bias_op == 1 && (lda != M || stride_ab != K * M)) return FDP_ERR_SHAPE;
